@@ -538,20 +538,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const GemmApply* ap
       offq[j] = (uint32_t)r * (uint32_t)g.ldq * 2u + c * 16u;
     }
   }
-  // Load j (0..7) of operand Q (or P) of stage `stage` into ring slot `slot`;
-  // stages past the end load the last one again (never read; it keeps every
-  // step's load count, and so the vmcnt bookkeeping, the same).
+  // Load j (0..7) of operand Q (or P) of stage `stage` (< KT) into ring slot `slot`.
   //
   // With a [K, N] Q the load is written as inline assembly, not the
   // compiler's builtin: the compiler then tracks no LDS-DMA writes and cannot
   // add vmcnt(0) waits in front of the transposing LDS reads, which it does
   // for every one of them (it cannot prove them disjoint from a pending DMA),
   // serializing the pipeline.  Completion is managed explicitly anyway: the
-  // vmcnt waits before the per-stage barriers, and the vmcnt(0) of the
-  // barrier before the epilogue.  The [N, K] form keeps the builtin, which
+  // vmcnt waits before the per-stage barriers.  No load is issued that no later
+  // step waits for, so none can land in the LDS once the epilogue reuses it (the
+  // barrier before the epilogue waits for no load by itself when the compiler
+  // tracks none).  The [N, K] form keeps the builtin, which
   // the compiler schedules a little tighter (about 120 cycles per stage).
   auto issue_load = [&](bool q, int slot, int64_t stage, int j) {
-    const int64_t k0 = (stage < KT ? stage : KT - 1) * BK;
+    const int64_t k0 = stage * BK;
     const uint16_t* base = q ? (kQKN ? Q + k0 * g.ldq : Q + k0) : P + k0;
     const uint16_t* dst = smem + slot * kSubTile +
                           ((q && kQKN) ? (wave * 16 + j * 2) * BN : (wave * 64 + j * 8) * BK);
@@ -669,34 +669,40 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const GemmApply* ap
   // One sub-step: 16 MFMAs on `cur`, the 8 fragments of `nxt` read from the
   // slots (rp, rq) at depth kk, and loads j0 .. j0 + 3 of (lq ? Q : P) of
   // stage lstage into slot ls_.
-  auto substep = [&](const Frags& cur, Frags& nxt, int rp, int rq, int kk, bool lq, int ls_,
-                     int64_t lstage, int j0) {
+  auto substep = [&](const Frags& cur, Frags& nxt, int rp, int rq, int kk, auto load, bool lq,
+                     int ls_, int64_t lstage, int j0) {
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
       mfma(n, cur);
       __builtin_amdgcn_sched_barrier(0);
       if (n < kReads) read(n, nxt, rp, rq, kk);
-      if (n >= 2 && n < 10 && (n & 1) == 0) issue_load(lq, ls_, lstage, j0 + ((n - 2) >> 1));
+      if constexpr (decltype(load)::value) {
+        if (n >= 2 && n < 10 && (n & 1) == 0) issue_load(lq, ls_, lstage, j0 + ((n - 2) >> 1));
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): next fragments in registers
   };
   // ps/qs: slots of stage t's P and Q; the slots of stage t + 1 and of P of
-  // stage t + 2 follow in ring order.
-  auto step = [&](int64_t t, int ps, auto next_tag) {
-    constexpr bool kNext = decltype(next_tag)::value;
+  // stage t + 2 follow in ring order.  kind: 0 with stages t + 1 and t + 2 to come,
+  // 1 the last but one (t = KT - 2), 2 the last (no loads, no barrier).
+  auto step = [&](int64_t t, int ps, auto kind) {
+    constexpr bool kNext = decltype(kind)::value < 2, kNext2 = decltype(kind)::value == 0;
     const int qs = ps + 1 == kSlots ? 0 : ps + 1;
     const int ps1 = qs + 1 == kSlots ? 0 : qs + 1;
     const int qs1 = ps1 + 1 == kSlots ? 0 : ps1 + 1;
     const int ps2 = qs1 + 1 == kSlots ? 0 : qs1 + 1;
-    substep(f0, f1, ps, qs, 1, true, qs1, t + 1, 4);   // Q of t + 1, loads 4..7
-    substep(f1, f0, ps, qs, 2, false, ps2, t + 2, 0);  // P of t + 2, loads 0..3
-    substep(f0, f1, ps, qs, 3, false, ps2, t + 2, 4);  // P of t + 2, loads 4..7
+    const std::bool_constant<kNext> l1;
+    const std::bool_constant<kNext2> l2;
+    substep(f0, f1, ps, qs, 1, l1, true, qs1, t + 1, 4);   // Q of t + 1, loads 4..7
+    substep(f1, f0, ps, qs, 2, l2, false, ps2, t + 2, 0);  // P of t + 2, loads 0..3
+    substep(f0, f1, ps, qs, 3, l2, false, ps2, t + 2, 4);  // P of t + 2, loads 4..7
     mfma(0, f1);
     mfma(1, f1);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kNext) {
-      __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): all but P of t + 2 landed for this wave
+      // vmcnt(8): all but P of t + 2 landed for this wave
+      __builtin_amdgcn_s_waitcnt(kNext2 ? 0x0F78 : 0x0F70);
       lds_barrier();
     }
 #pragma unroll
@@ -706,36 +712,51 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const GemmApply* ap
       if constexpr (kNext) {
         if (n - 2 < kReads) read(n - 2, f0, ps1, qs1, 0);
         // Q of t + 2 into the freed P slot of t, loads 0..3
-        if (n >= 6 && n < 14 && (n & 1) == 0) issue_load(true, ps, t + 2, (n - 6) >> 1);
+        if constexpr (kNext2) {
+          if (n >= 6 && n < 14 && (n & 1) == 0) issue_load(true, ps, t + 2, (n - 6) >> 1);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kNext) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   };
 
+  // The last two steps load only what a later step computes: re-loading the last
+  // stage instead, to keep one load count, cost 0.9-6% of a Newton-Schulz chain (one
+  // 200 x 96 gradient 201 -> 190 us, 42 matrices of 3072 x 6144 39.1 -> 38.8 ms a step).
+  //
   // Prologue: P0 Q0 P1 in full and the first half of Q1 (slots 0..3), then
   // stage 0 is waited for and its first fragments read.
 #pragma unroll
   for (int j = 0; j < 8; ++j) issue_load(false, 0, 0, j);
 #pragma unroll
   for (int j = 0; j < 8; ++j) issue_load(true, 1, 0, j);
+  if (KT > 1) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) issue_load(false, 2, 1, j);
+    for (int j = 0; j < 8; ++j) issue_load(false, 2, 1, j);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) issue_load(true, 3, 1, j);
-  __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): P0 and Q0 landed for this wave
+    for (int j = 0; j < 4; ++j) issue_load(true, 3, 1, j);
+    __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): P0 and Q0 landed for this wave
+  } else {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  }
   lds_barrier();
 #pragma unroll
   for (int n = 0; n < kReads; ++n) read(n, f0, 0, 1, 0);
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 
   int ps = 0;
-  for (int64_t t = 0; t + 1 < KT; ++t) {
-    step(t, ps, std::true_type{});
-    ps = ps + 2 >= kSlots ? ps + 2 - kSlots : ps + 2;
+  auto advance = [&]() { ps = ps + 2 >= kSlots ? ps + 2 - kSlots : ps + 2; };
+  for (int64_t t = 0; t + 2 < KT; ++t) {
+    step(t, ps, std::integral_constant<int, 0>{});
+    advance();
   }
-  step(KT - 1, ps, std::false_type{});
-  __syncthreads();  // all fragment reads and trailing loads done before the epilogue reuses the LDS
+  if (KT > 1) {
+    step(KT - 2, ps, std::integral_constant<int, 1>{});
+    advance();
+  }
+  step(KT - 1, ps, std::integral_constant<int, 2>{});
+  __syncthreads();  // every wave's fragment reads done before the epilogue reuses the LDS
 
   // ---- epilogue ------------------------------------------------------------
   if constexpr (kApply) {
