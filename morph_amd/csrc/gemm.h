@@ -1,9 +1,12 @@
-// Library-internal entry of the batched bf16 GEMM (gemm.hip).
+// Library-internal entry of the batched bf16 GEMM (gemm.hip).  M and N are
+// multiples of kGemmEdge here (the exported entry keeps its 256).
 #pragma once
 
 #include <stdint.h>
 
 namespace morph {
+
+constexpr int kGemmEdge = 64;  // the smallest tile edge
 
 // morph_gemm_nt_bf16 with an optional per-matrix factor: when bscale is not
 // null, matrix b of the batch uses alpha * bscale[b] and beta * bscale[b]
@@ -18,11 +21,16 @@ __attribute__((visibility("hidden"))) int gemm_nt_bf16_scaled(
     int64_t stride_c, int64_t stride_ct, float alpha, float beta, const float* bscale,
     float diag, int flags, void* stream);
 
+// Estimated time in us of one product (M, N multiples of kGemmEdge), by the rule that
+// picks its tile: for choosing how far to pad the operands.
+__attribute__((visibility("hidden"))) double gemm_us(int64_t M, int64_t N, int64_t K,
+                                                     int64_t batch, bool symmetric, bool has_d);
+
 // The Muon master update carried by the last Newton-Schulz product X' = B' X
 // (gemm_kn_apply): instead of storing X', the epilogue rounds each element to
 // bf16 as the store would and updates matrix b's FP32 parameter in place,
 // p = fma(bf16(X') * scale[b], neg_lr, p * decay), with X' in p's layout.  X
-// is [m, n] with no padding (m, n multiples of the 256 tile); p[b] is [m, n]
+// is [m, n] with no padding (m, n multiples of kGemmEdge); p[b] is [m, n]
 // (row length n), or [n, m] (row length m) when transposed[b], 16-byte aligned.
 constexpr int kGemmMaxApply = 64;
 struct GemmApply {

@@ -31,7 +31,7 @@
 // per-block partial sums f64; per-matrix 1/den, 1/den^2, den f32;
 // X0/X1 [count][Mp][Np] (iterations alternate: X' = B' X reads all of X as its
 // [K, N] operand, so it cannot overwrite it), A and B' [count][Mp][Mp], bf16,
-// with m = min(rows, cols), n = max, Mp/Np rounded up to the GEMM tile.  prepare
+// with m = min(rows, cols), n = max, Mp/Np rounded up to a GEMM tile edge (pad_multiple).  prepare
 // writes X0 including its zero padding (pad_zero_kernel) and every product
 // rewrites its whole padded output, so no call depends on an earlier one.  The
 // zero padding is exact for Newton-Schulz: padded rows of X give zero rows and
@@ -99,15 +99,33 @@ struct Layout {
   size_t off_part, off_scale, off_x0, off_x1, off_a, off_b, total;
 };
 
-Layout make_layout(int64_t rows, int64_t cols, int64_t count) {
+// How far m and n are rounded up: the multiple (a GEMM tile edge) with the fastest
+// Newton-Schulz iteration.  More padding can allow a larger tile; less is less work,
+// and none lets the last product carry the update (10 us: no padding launch, no
+// finish pass).  The results do not depend on it (zero padding is exact).
+int64_t pad_multiple(int64_t m, int64_t n, int64_t count) {
+  int64_t best = 0;
+  double best_us = 0.0;
+  for (int64_t u = 256; u >= kGemmEdge; u /= 2) {
+    const int64_t mp = round_up(m, u), np = round_up(n, u);
+    const double us = 5.0 * (gemm_us(mp, mp, np, count, true, false) +
+                             gemm_us(mp, mp, mp, count, true, true) +
+                             gemm_us(mp, np, mp, count, false, false)) +
+                      (mp == m && np == n ? 0.0 : 10.0);
+    if (best == 0 || us < best_us) best = u, best_us = us;
+  }
+  return best;
+}
+
+Layout make_layout(int64_t rows, int64_t cols, int64_t count, int64_t multiple) {
   Layout L;
   L.rows = rows;
   L.cols = cols;
   L.count = count;
   L.m = rows < cols ? rows : cols;
   L.n = rows < cols ? cols : rows;
-  L.mp = round_up(L.m, MORPH_GEMM_TILE_M);
-  L.np = round_up(L.n, MORPH_GEMM_TILE_N);  // also a multiple of the K tile (64)
+  L.mp = round_up(L.m, multiple);
+  L.np = round_up(L.n, multiple);  // also a multiple of the K stage (64)
   L.ldn = L.np + kRowPad;
   L.ldm = L.mp + kRowPad;
   L.numel = rows * cols;
@@ -130,6 +148,16 @@ Layout make_layout(int64_t rows, int64_t cols, int64_t count) {
   L.off_b = take((size_t)count * L.mp * L.ldm * 2);
   L.total = off;
   return L;
+}
+
+Layout make_layout(int64_t rows, int64_t cols, int64_t count) {
+  return make_layout(rows, cols, count,
+                     pad_multiple(std::min(rows, cols), std::max(rows, cols), count));
+}
+
+// The workspace a batch may ask for, whichever multiple it is padded to: the largest.
+size_t workspace_bytes_for(int64_t rows, int64_t cols, int64_t count) {
+  return make_layout(rows, cols, count, MORPH_GEMM_TILE_M).total;
 }
 
 template <int kLanes = kBlock>
@@ -568,7 +596,7 @@ using namespace morph;
 
 extern "C" size_t morph_muon_workspace_bytes(int64_t rows, int64_t cols, int count) {
   if (rows <= 0 || cols <= 0 || count <= 0) return 0;
-  return make_layout(rows, cols, count).total;
+  return workspace_bytes_for(rows, cols, count);
 }
 
 namespace {
@@ -598,7 +626,8 @@ int setup(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
         return MORPH_EINVAL;
   }
   const Layout L = make_layout(rows, cols, count > 0 ? count : 1);
-  if (workspace == nullptr || workspace_bytes < L.total) return MORPH_EWORKSPACE;
+  if (workspace == nullptr || workspace_bytes < workspace_bytes_for(rows, cols, L.count))
+    return MORPH_EWORKSPACE;
   if (reinterpret_cast<uintptr_t>(workspace) % 256) return MORPH_EINVAL;
   // grid x of the tile passes and of apply_flat_kernel (the most blocks of the flat passes)
   if (L.tiles > INT32_MAX || L.atiles > INT32_MAX ||

@@ -137,7 +137,8 @@ def ns_flops(rows, cols, count, steps=NS_STEPS):
 def ns_executed_flops(rows, cols, count, steps=NS_STEPS):
     """FLOPs the MFMAs execute: the symmetric products (A = X X^T, B' = c A A + b A + a I)
     compute only the upper triangle of their 256 x 256 tiles, X' = B' X all of them; the
-    operands are zero-padded to tile multiples (Mp, Np)."""
+    operands are zero-padded to tile multiples (Mp, Np).  An upper bound for small batches,
+    which run smaller tiles with less padding."""
     m, n = min(rows, cols), max(rows, cols)
     mp, np_ = -(-m // 256) * 256, -(-n // 256) * 256
     t, tn = mp // 256, np_ // 256

@@ -67,6 +67,52 @@ def test_gemm_q_kn_equals_the_nt_form_bit_for_bit(b, M, N, K):
     assert ((C - exact).abs() <= 2 ** -8 * exact.abs() + 1e-6 * K * mag + 1e-30).all()
 
 
+@pytest.mark.parametrize("M,N,K,batches", [(512, 512, 4096, (3, 12, 64)), (256, 512, 320, (2, 300)),
+                                           (256, 256, 192, (1, 512)), (256, 256, 128, (1, 512))])
+def test_gemm_tile_edges_give_the_same_bits(M, N, K, batches):
+    """The batch decides the tile edge (64, 128 or 256: fewer tiles, smaller ones), never the
+    bits: every output is one accumulator's sum over K in the same order, rounded once.  The
+    smallest batch is checked against the float64 product, the larger ones against it; with
+    and without D, factors and Ct, [K, N] operands, and symmetric with mirror tiles."""
+    P, Q, D = rand_bf16((4, M, K), 1), rand_bf16((4, N, K), 2), rand_bf16((4, M, N), 3)
+    S = rand_bf16((4, M, M), 4)
+    forms = {}
+    for b in batches:
+        rep = lambda t: t.repeat((-(-b // 4), 1, 1))[:b].contiguous().to(DEV)  # noqa: E731
+        Pd, Qd, Dd = rep(P), rep(Q), rep(D)
+        Sd = rep(S + S.transpose(1, 2))
+        Qkn = Qd.transpose(1, 2).contiguous()
+        ct = torch.empty((b, N, M), dtype=torch.bfloat16, device=DEV)
+        got = dict(nt=muon.gemm_nt(Pd, Qd), ntd=muon.gemm_nt(Pd, Qd, Dd, 2.0315, -4.775, out_t=ct),
+                   ct=ct, kn=muon.gemm_nt(Pd, Qkn, q_kn=True),
+                   knd=muon.gemm_nt(Pd, Qkn, Dd, 3.0, -0.5, q_kn=True),
+                   sym=muon.gemm_nt(Pd, Pd, symmetric=True),
+                   symd=muon.gemm_nt(Pd, Pd, Sd, 2.0315, -4.775, symmetric=True))
+        for name, out in got.items():
+            first = forms.setdefault(name, out[:4].clone())
+            n = min(len(first), b)
+            assert torch.equal(out[:n].view(torch.int16), first[:n].view(torch.int16)), (name, b)
+            assert torch.equal(out[-1].view(torch.int16), out[(b - 1) % 4].view(torch.int16)), (name, b)
+    exact = P[0].double() @ Q[0].double().t()
+    mag = P[0].double().abs() @ Q[0].double().abs().t()
+    err = (forms["nt"][0].cpu().double() - exact).abs()
+    assert (err <= 2 ** -8 * exact.abs() + 1e-6 * K * mag + 1e-30).all()
+    assert torch.equal(forms["sym"][0], forms["sym"][0].t())
+
+
+@pytest.mark.parametrize("shape,counts", [((330, 700), (1, 32, 64)), ((900, 450), (1, 8, 33)),
+                                          ((70, 45), (1, 40)), ((256, 320), (1, 64))])
+def test_padding_and_tiles_do_not_change_the_bits(shape, counts):
+    """A matrix's Newton-Schulz result, alone or among many: the batch's size decides how far
+    the operands are padded (64, 128 or 256) and the tile edges, and none of it the bits."""
+    gen = torch.Generator().manual_seed(9)
+    gs = [(torch.randn(shape, generator=gen) * 1e-3).to(DEV) for _ in range(max(counts))]
+    ref = [muon.orthogonalize(g) for g in gs[:3]]
+    for n in counts[1:]:
+        for a, b in zip(ref, muon.orthogonalize(gs[:n])):
+            assert_same_bits(a.cpu().numpy(), b.cpu().numpy(), f"batch of {n}")
+
+
 @pytest.mark.parametrize("alpha", [1 + 2 ** -8, 1 + 3 * 2 ** -8, 1 / 3, -0.7, 2.0 ** -140, 7.5e37])
 def test_gemm_output_rounding_is_round_to_nearest_even(alpha):
     """C = alpha * I Q^T is one fp32 product alpha * q rounded once to bf16.  With q a
