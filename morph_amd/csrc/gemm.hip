@@ -975,18 +975,25 @@ void launch_apply(bool scaled, unsigned grid, hipStream_t s, const GemmArgs& g,
 // constants measured on the device (one MI355X, 256 CUs) over 1 to 42 operands of
 // 256 x 256 to 3072 x 6144.  256: rounds of one tile per CU, a stage 1.0 us when few
 // CUs work and 1.45 us on a full chip (its clock falls), 8.5 us of prologue and
-// epilogue (15 with D).  128: n tiles on the fullest CU, two at a time, whose
+// epilogue (15 with D, 30 with the update, whose masters every CU moves at the same
+// time).  128: n tiles on the fullest CU, two at a time, whose
 // prologues and epilogues overlap.  64: latency up to a tile per CU, then three at a
 // time, bound by the LDS (a 32 x 32 block per wave reads a fragment per MFMA operand).
-double launch_us(int ts, int64_t tiles, int64_t kt, bool has_d) {
+enum class Epilogue { kPlain, kWithD, kUpdate };
+
+double launch_us(int ts, int64_t tiles, int64_t kt, Epilogue e) {
+  const bool d = e == Epilogue::kWithD, up = e == Epilogue::kUpdate;
   const double q = (double)tiles / 256.0, n = std::ceil(q);
   if (ts == 256) {
     const double full = q / n;
-    return n * ((double)kt * (1.0 + 0.45 * full * full) + (has_d ? 15.0 : 8.5));
+    return n * ((double)kt * (1.0 + 0.45 * full * full) + (d ? 15.0 : up ? 30.0 : 8.5));
   }
   if (ts == 128) {
-    const double stage = n <= 1.0 ? 0.55 : n <= 2.0 ? 0.8 : 0.45 * n + 0.1;
-    return (double)kt * stage + n * (has_d ? 2.3 : 1.3) + 2.0;
+    const double stage = n <= 1.0   ? 0.55
+                         : n <= 2.0 ? 0.8
+                         : n <= 8.0 ? 0.45 * n + 0.1
+                                    : 0.5 * n - 0.3;
+    return (double)kt * stage + n * (d ? 2.3 : up ? 6.0 : 1.3) + 2.0;
   }
   return (double)kt * std::max(0.22, 0.24 * q) + 3.0;
 }
@@ -1001,14 +1008,15 @@ struct Choice {
 // 16, rounded once.  Measured, us per launch with edges 256 / 128 / 64:
 //   A = X X^T, one 768 x 2048: 39 / 16 / 10; twelve: 41 / 24 / 29; thirty-six: 55 / 54 / 70;
 //   one 3072 x 6144: 102 / 75 / 120; three: 146 / 179 / 352;
-//   X' = B' X, one 3072 x 6144: 128 / 114 / 168; three: 288 / 314 / 505.
-Choice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool symmetric, bool has_d) {
+//   X' = B' X, one 3072 x 6144: 128 / 114 / 168; three: 288 / 314 / 505;
+//   its update, thirty-six 768 x 2048: 201 / 182 (256 / 128).
+Choice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool symmetric, Epilogue e) {
   Choice best{0, 0.0};
   for (int ts = 256; ts >= 64; ts /= 2) {
     if (M % ts || N % ts) continue;
     const int64_t tm = M / ts, tn = N / ts;
     const int64_t tiles = batch * (symmetric ? tm * (tm + 1) / 2 : tm * tn);
-    const double us = launch_us(ts, tiles, K / BK, has_d);
+    const double us = launch_us(ts, tiles, K / BK, e);
     if (best.ts == 0 || us < best.us) best = Choice{ts, us};
   }
   return best;
@@ -1018,7 +1026,7 @@ Choice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool symmetri
 }  // namespace morph
 
 double morph::gemm_us(int64_t M, int64_t N, int64_t K, int64_t batch, bool symmetric, bool has_d) {
-  return choose_tile(M, N, K, batch, symmetric, has_d).us;
+  return choose_tile(M, N, K, batch, symmetric, has_d ? Epilogue::kWithD : Epilogue::kPlain).us;
 }
 
 int morph::gemm_nt_bf16_scaled(const uint16_t* P, const uint16_t* Q, const uint16_t* D,
@@ -1074,7 +1082,8 @@ int morph::gemm_nt_bf16_scaled(const uint16_t* P, const uint16_t* Q, const uint1
     const auto st = span(Ct, stride_ct, N, ldct, M);
     if (meet(st, sp) || meet(st, sq) || meet(st, sc)) return MORPH_EINVAL;
   }
-  const int ts = choose_tile(M, N, K, batch, symmetric, D != nullptr).ts;
+  const int ts =
+      choose_tile(M, N, K, batch, symmetric, D != nullptr ? Epilogue::kWithD : Epilogue::kPlain).ts;
   const int64_t tm = M / ts, tn = N / ts;
   const int64_t per = symmetric ? tm * (tm + 1) / 2 : tm * tn;
   const int64_t total = batch * per;
@@ -1113,7 +1122,7 @@ int morph::gemm_kn_apply(const uint16_t* P, const uint16_t* Q, int64_t M, int64_
   // 32-bit offsets inside a tile: 255 rows of the widest row length
   constexpr int64_t kMaxLd = int64_t(1) << 23;
   if (ldp > kMaxLd || ldq > kMaxLd || M > kMaxLd || N > kMaxLd) return MORPH_ERANGE;
-  const int ts = choose_tile(M, N, K, batch, false, false).ts;
+  const int ts = choose_tile(M, N, K, batch, false, Epilogue::kUpdate).ts;
   const int64_t tm = M / ts, tn = N / ts, per = tm * tn, total = batch * per;
   const int64_t grid = (total + 7) / 8 * 8;
   if (grid > (int64_t(1) << 31) - 1) return MORPH_ERANGE;
