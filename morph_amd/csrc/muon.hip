@@ -44,6 +44,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "muon_small.h"
 
 namespace morph {
 namespace {
@@ -677,6 +678,52 @@ MatPtrs pointers(const morph_muon_matrix* mats, int count, int64_t rows, int64_t
   return m;
 }
 
+static_assert(kSmallMaxMats >= kMaxMats, "a whole batch in one small launch");
+
+// Small operands run the one-workgroup-per-matrix kernels (muon_small.hip).  With no
+// iterations there is no chain: those keep the general passes.
+bool takes_small(const Layout& L, const morph_muon_hp* hp) {
+  return hp->ns_steps >= 1 && small_fits(L.m, L.n);
+}
+
+// mats (nullable): the batch's descriptors, needed by prepare and by an updating chain.
+SmallBatch small_batch(const Bufs& W, const morph_muon_matrix* mats, int count) {
+  const Layout& L = W.L;
+  SmallBatch b;
+  b.tall = 0;
+  b.form = reinterpret_cast<uint32_t*>(W.part);
+  b.x0 = W.X[0];
+  b.scale = W.scale;
+  b.stride = L.mp * L.ldn;
+  b.m = (int32_t)L.m;
+  b.n = (int32_t)L.n;
+  b.count = count;
+  for (int i = 0; mats != nullptr && i < count; ++i) {
+    b.grad[i] = mats[i].grad;
+    b.mom[i] = mats[i].momentum;
+    b.mom_out[i] = mats[i].momentum_out != nullptr ? mats[i].momentum_out : mats[i].momentum;
+    b.param[i] = mats[i].param;
+    if (!stored_is_x(mats[i], L.rows, L.cols)) b.tall |= uint64_t(1) << i;
+  }
+  return b;
+}
+
+int run_small_chain(const Bufs& W, const morph_muon_matrix* mats, int count,
+                    const morph_muon_hp* hp, SmallOut out, hipStream_t s) {
+  SmallChain c;
+  c.a = hp->a;
+  c.b = hp->b;
+  c.c = hp->c;
+  c.steps = hp->ns_steps;
+  c.x = W.X[hp->ns_steps & 1];  // where finish looks for it
+  c.ldx = W.L.ldn;
+  c.decay = hp->decay;
+  c.neg_lr = hp->neg_lr;
+  for (int i = 0; mats != nullptr && i < count; ++i)
+    c.scale[i] = mats[i].transposed ? hp->update_scale_transposed : hp->update_scale;
+  return small_chain(small_batch(W, mats, count), c, out, s);
+}
+
 int prepare(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
             const morph_muon_hp* hp, void* workspace, size_t workspace_bytes, bool orth_only,
             uint32_t* found_inf, void* stream) {
@@ -685,6 +732,9 @@ int prepare(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols
   if (rc || count == 0) return rc;
   const Layout& L = W.L;
   hipStream_t s = as_stream(stream);
+  if (takes_small(L, hp))
+    return small_prepare(small_batch(W, mats, count), orth_only, hp->momentum_weight,
+                         hp->nesterov_weight, found_inf, s);
   int n_all, n_flat, n_tiled;
   const MatPtrs mp_ = pointers(mats, count, rows, cols, Orient::kAll, &n_all);
   const MatPtrs flat = pointers(mats, count, rows, cols, Orient::kStored, &n_flat);
@@ -739,8 +789,8 @@ bool can_fuse_update(const morph_muon_matrix* mats, int count, const Layout& L) 
   return true;
 }
 
-// fuse: the batch's matrices, whose parameter update the last product carries in
-// place of writing X (can_fuse_update must hold); nullptr: X is written.
+// fuse: the batch's matrices, whose parameter update the last product (or the small
+// chain) carries in place of writing X (can_fuse_update must hold); nullptr: X is written.
 int newton_schulz(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp,
                   void* workspace, size_t workspace_bytes, void* stream,
                   const morph_muon_matrix* fuse = nullptr) {
@@ -748,6 +798,10 @@ int newton_schulz(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp
   int rc = setup(nullptr, count, rows, cols, hp, workspace, workspace_bytes, false, false, &W);
   if (rc || count == 0) return rc;
   const Layout& L = W.L;
+  if (takes_small(L, hp))
+    return run_small_chain(W, fuse, count, hp,
+                           fuse != nullptr ? SmallOut::kApply : SmallOut::kStore,
+                           as_stream(stream));
   const int64_t sx = L.mp * L.ldn, ss = L.mp * L.ldm;
   const int64_t n = L.ldn, m = L.ldm;  // leading dimensions
   int cur = 0;
@@ -841,7 +895,7 @@ int newton_schulz_finish(const morph_muon_matrix* mats, int count, int64_t rows,
   Bufs W;
   int rc = setup(mats, count, rows, cols, hp, workspace, workspace_bytes, true, false, &W);
   if (rc || count == 0) return rc;
-  if (hp->ns_steps >= 1 && can_fuse_update(mats, count, W.L))
+  if (hp->ns_steps >= 1 && (takes_small(W.L, hp) || can_fuse_update(mats, count, W.L)))
     return newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, mats);
   rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream);
   if (!rc) rc = finish(mats, count, rows, cols, hp, workspace, workspace_bytes, false, stream);
@@ -899,7 +953,13 @@ extern "C" int morph_muon_orthogonalize(const morph_muon_matrix* mats, int count
                                         int64_t cols, const morph_muon_hp* hp, void* workspace,
                                         size_t workspace_bytes, void* stream) {
   int rc = prepare(mats, count, rows, cols, hp, workspace, workspace_bytes, true, nullptr, stream);
-  if (!rc) rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream);
+  if (rc || count == 0) return rc;
+  Bufs W;
+  rc = setup(mats, count, rows, cols, hp, workspace, workspace_bytes, true, false, &W);
+  if (rc) return rc;
+  if (takes_small(W.L, hp))
+    return run_small_chain(W, mats, count, hp, SmallOut::kExtract, as_stream(stream));
+  rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream);
   if (!rc) rc = finish(mats, count, rows, cols, hp, workspace, workspace_bytes, true, stream);
   return rc;
 }

@@ -146,8 +146,20 @@ def ns_executed_flops(rows, cols, count, steps=NS_STEPS):
     return 2 * count * steps * macs
 
 
-def _prepare(mats, rows, cols, hp, orth_only, stream, workspaces, found_inf=None, first=0):
-    """Enqueue prepare for up to 64 matrices per batch; returns the batches for _complete.
+def _batch(mats, rows, cols, stream, workspaces, index):
+    """The descriptors of up to 64 matrices and their workspace (see _prepare)."""
+    ws = workspaces.get(rows, cols, len(mats), mats[0][0][0].device, index, stream)
+    arr = (MuonMatrix * len(mats))()
+    for d, ((p, g, m, m_out), transposed) in zip(arr, mats):
+        d.grad, d.param = g.data_ptr(), p.data_ptr()
+        d.momentum = m.data_ptr() if m is not None else None
+        d.momentum_out = m_out.data_ptr() if m_out is not None else None
+        d.transposed = transposed
+    return arr, len(mats), ws
+
+
+def _prepare(mats, rows, cols, hp, stream, workspaces, found_inf=None, first=0):
+    """Enqueue a Muon step's prepare for up to 64 matrices per batch; returns the batches.
 
     mats: [((param, grad, momentum, momentum_out), transposed)], each stored
     [rows, cols], or [cols, rows] when transposed.  found_inf: optional device
@@ -157,28 +169,20 @@ def _prepare(mats, rows, cols, hp, orth_only, stream, workspaces, found_inf=None
     L = lib()
     batches = []
     for k, start in enumerate(range(0, len(mats), 64)):
-        chunk = mats[start:start + 64]
-        ws = workspaces.get(rows, cols, len(chunk), chunk[0][0][0].device, first + k, stream)
-        arr = (MuonMatrix * len(chunk))()
-        for i, ((p, g, m, m_out), transposed) in enumerate(chunk):
-            arr[i].grad, arr[i].param = g.data_ptr(), p.data_ptr()
-            arr[i].momentum = m.data_ptr() if m is not None else None
-            arr[i].momentum_out = m_out.data_ptr() if m_out is not None else None
-            arr[i].transposed = transposed
+        arr, count, ws = _batch(mats[start:start + 64], rows, cols, stream, workspaces, first + k)
         flag = ctypes.c_void_p(found_inf.data_ptr()) if found_inf is not None else None
-        check(L.morph_muon_prepare(arr, len(chunk), rows, cols, ctypes.byref(hp), int(orth_only),
+        check(L.morph_muon_prepare(arr, count, rows, cols, ctypes.byref(hp), 0,
                                    ctypes.c_void_p(ws.data_ptr()), ws.numel(), flag,
                                    stream_handle(stream)))
-        batches.append((arr, len(chunk), rows, cols, hp, orth_only, ws))
+        batches.append((arr, count, rows, cols, hp, ws))
     return batches
 
 
 def _finish_range(batch, first, n, stream):
-    """The parameter update (or U into param) of matrices first .. first + n - 1 of a
-    batch _prepare enqueued."""
-    arr, count, rows, cols, hp, orth_only, ws = batch
-    check(lib().morph_muon_finish_range(arr, count, rows, cols, ctypes.byref(hp), int(orth_only),
-                                        first, n, ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+    """The parameter update of matrices first .. first + n - 1 of a batch _prepare enqueued."""
+    arr, count, rows, cols, hp, ws = batch
+    check(lib().morph_muon_finish_range(arr, count, rows, cols, ctypes.byref(hp), 0, first, n,
+                                        ctypes.c_void_p(ws.data_ptr()), ws.numel(),
                                         stream_handle(stream)))
 
 
@@ -186,19 +190,19 @@ def _chains(batches, stream, timer=None, with_update=False):
     """The Newton-Schulz chain of every batch _prepare enqueued.
 
     timer: optional list; (start_event, end_event, dense flops, executed flops) around
-    each NS chain.  with_update: the chain of a Muon-step batch also applies the
-    parameter update (morph_muon_newton_schulz_finish: in its last product's epilogue
-    where the shape allows), so no finish follows; orthogonalize batches are chains only.
+    each NS chain.  with_update: the chain also applies the parameter update
+    (morph_muon_newton_schulz_finish: in its last product's epilogue where the shape
+    allows), so no finish follows.
     """
     L = lib()
     sh = stream_handle(stream)
-    for arr, count, rows, cols, hp, orth_only, ws in batches:
+    for arr, count, rows, cols, hp, ws in batches:
         wsp, wsn = ctypes.c_void_p(ws.data_ptr()), ws.numel()
         if timer is not None:
             s = stream or torch.cuda.current_stream()
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record(s)
-        if with_update and not orth_only:
+        if with_update:
             check(L.morph_muon_newton_schulz_finish(arr, count, rows, cols, ctypes.byref(hp), wsp,
                                                     wsn, sh))
         else:
@@ -207,19 +211,6 @@ def _chains(batches, stream, timer=None, with_update=False):
             e1.record(s)
             timer.append((e0, e1, ns_flops(rows, cols, count, hp.ns_steps),
                           ns_executed_flops(rows, cols, count, hp.ns_steps)))
-
-
-def _complete(batches, stream, timer=None):
-    """Newton-Schulz chains and the finish of every batch _prepare enqueued: a Muon
-    step's update rides on its chain (morph_muon_newton_schulz_finish), orthogonalize's
-    U goes into param by the finish pass."""
-    _chains(batches, stream, timer, with_update=True)
-    L = lib()
-    sh = stream_handle(stream)
-    for arr, count, rows, cols, hp, orth_only, ws in batches:
-        if orth_only:
-            check(L.morph_muon_finish(arr, count, rows, cols, ctypes.byref(hp), 1,
-                                      ctypes.c_void_p(ws.data_ptr()), ws.numel(), sh))
 
 
 def _check_matrix(t, name):
@@ -241,11 +232,13 @@ def orthogonalize(gradients, steps=NS_STEPS, stream=None, workspaces=_WORKSPACES
         _check_matrix(g, "gradient")
         outs.append(torch.empty_like(g))
     items = [(o, g, None, None) for o, g in zip(outs, gs)]
-    batches = []
+    L, hp, sh, k = lib(), _hp(steps=steps), stream_handle(stream), 0
     for (rows, cols), group in _by_shape(items).items():
-        batches += _prepare(group, rows, cols, _hp(steps=steps), True, stream, workspaces,
-                            first=len(batches))
-    _complete(batches, stream)
+        for start in range(0, len(group), 64):
+            arr, count, ws = _batch(group[start:start + 64], rows, cols, stream, workspaces, k)
+            check(L.morph_muon_orthogonalize(arr, count, rows, cols, ctypes.byref(hp),
+                                             ctypes.c_void_p(ws.data_ptr()), ws.numel(), sh))
+            k += 1
     return outs[0] if single else outs
 
 
@@ -290,10 +283,10 @@ def muon_step(params, grads, momenta, lr, weight_decay, steps=NS_STEPS, stream=N
     batches = []
     for (rows, cols), group in _by_shape(items).items():
         batches += _prepare(group, rows, cols, _step_hp(rows, cols, lr, weight_decay, steps),
-                            False, stream, workspaces, found_inf, first=len(batches))
+                            stream, workspaces, found_inf, first=len(batches))
     if gate is not None:
         gate()
-    _complete(batches, stream, timer)
+    _chains(batches, stream, timer, with_update=True)
 
 
 def _muon_grad(g, p, device):
@@ -561,9 +554,8 @@ class HybridMuonAdamW:
             batches = []
             for (rows, cols), group in _by_shape(items).items():
                 batches += _prepare(group, rows, cols,
-                                    _step_hp(rows, cols, self.lr, self.weight_decay), False,
-                                    stream, self._workspaces, self._flag,
-                                    first=nbatch + len(batches))
+                                    _step_hp(rows, cols, self.lr, self.weight_decay), stream,
+                                    self._workspaces, self._flag, first=nbatch + len(batches))
             nbatch += len(batches)
             ns.wait_stream(stream)
             self._workspaces.note_stream(ns)

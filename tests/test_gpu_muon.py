@@ -113,6 +113,84 @@ def test_padding_and_tiles_do_not_change_the_bits(shape, counts):
             assert_same_bits(a.cpu().numpy(), b.cpu().numpy(), f"batch of {n}")
 
 
+# (m, n) at the edges of the one-workgroup path: 32-row blocks, the largest n that the LDS
+# takes for 1, 2, 3 and 4 of them, odd and single rows; wide: zero columns past that n.
+SMALL = [(1, 1, 2600), (5, 33, 2600), (31, 2496, 2600), (33, 65, 1300), (64, 1184, 1300),
+         (70, 75, 800), (96, 736, 800), (97, 101, 700), (128, 480, 700), (100, 256, 700)]
+
+
+@pytest.mark.parametrize("m,n,wide", SMALL)
+def test_small_matrices_equal_the_general_chain_bit_for_bit(m, n, wide):
+    """A small matrix's whole chain runs in one workgroup; the same matrix with zero columns
+    appended is too wide for that and takes the general products.  Dyadic values make the FP64
+    norm exact in any order, so the results must be the same bits, in both orientations."""
+    gen = torch.Generator().manual_seed(m * n)
+    g = torch.randint(-511, 512, (m, n), generator=gen).float() * 2.0 ** -14
+    g[0, 0] = 2.0 ** -5
+    padded = torch.zeros(m, wide)
+    padded[:, :n] = g
+    want = muon.orthogonalize(padded.to(DEV)).cpu()
+    got = muon.orthogonalize(g.to(DEV)).cpu()
+    assert_same_bits(got.numpy(), want[:, :n].numpy(), "stored")
+    tall = muon.orthogonalize(g.t().contiguous().to(DEV)).cpu()
+    assert_same_bits(tall.numpy(), got.t().contiguous().numpy(), "transposed")
+
+
+@pytest.mark.parametrize("shape", [(64, 192), (65, 33)])
+@pytest.mark.parametrize("at", [0, 1, 2, 3, 1025, -1])
+def test_small_prepare_flags_every_element(shape, at):
+    g = torch.zeros(shape)
+    g.view(-1)[at] = float("inf")
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    p, m = torch.zeros(shape, device=DEV), torch.zeros(shape, device=DEV)
+    for grad, want in ((torch.ones(shape), 0), (g, 1)):
+        muon.muon_step([p], [grad.to(DEV)], [m], .02, .01, found_inf=flag)
+        assert flag.item() == want
+
+
+@pytest.mark.parametrize("m,n", [(96, 200), (33, 65), (7, 50), (128, 480)])
+@pytest.mark.parametrize("steps", [1, 2, 5])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_small_update_equals_the_finish_pass(m, n, steps, offset):
+    """The small chain's own update against its stored X and the finish pass, both orientations
+    in one batch, parameters on and off 16 bytes; the gate's flag and the momentum too."""
+    import ctypes
+    from morph_amd import _lib
+    L = _lib.lib()
+    gen = torch.Generator().manual_seed(m + n)
+    shapes = [(m, n), (n, m), (n, m)]
+    place = lambda t: torch.cat([torch.zeros(offset), t.reshape(-1)]).to(DEV)[offset:].view(t.shape)  # noqa: E731
+    p0, m0, g = ([place(torch.randn(s, generator=gen) * k) for s in shapes] for k in (.02, 1e-3, 1e-3))
+    hp = muon._step_hp(m, n, .02, .01, steps)
+    ws = torch.full((L.morph_muon_workspace_bytes(m, n, 3),), 0xFF, dtype=torch.uint8, device=DEV)
+    wsp, sh, hpp = ctypes.c_void_p(ws.data_ptr()), _lib.stream_handle(), ctypes.byref(hp)
+    results = []
+    for fused in (True, False):
+        p, mom = [place(t.cpu()) for t in p0], [place(t.cpu()) for t in m0]
+        flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+        arr = (_lib.MuonMatrix * 3)()
+        for i in range(3):
+            arr[i].grad, arr[i].momentum, arr[i].param = (g[i].data_ptr(), mom[i].data_ptr(),
+                                                          p[i].data_ptr())
+            arr[i].transposed = int(shapes[i] != (m, n))
+        _lib.check(L.morph_muon_prepare(arr, 3, m, n, hpp, 0, wsp, ws.numel(),
+                                        ctypes.c_void_p(flag.data_ptr()), sh))
+        if fused:
+            _lib.check(L.morph_muon_newton_schulz_finish(arr, 3, m, n, hpp, wsp, ws.numel(), sh))
+        else:
+            _lib.check(L.morph_muon_newton_schulz(3, m, n, hpp, wsp, ws.numel(), sh))
+            _lib.check(L.morph_muon_finish(arr, 3, m, n, hpp, 0, wsp, ws.numel(), sh))
+        assert flag.item() == 0
+        results.append((p, mom))
+    for i in range(3):
+        assert torch.equal(results[0][0][i], results[1][0][i]), i
+        assert torch.equal(results[0][1][i], results[1][1][i]), i
+        assert not torch.equal(results[0][0][i], p0[i])
+        want = m0[i].cpu() + 0  # momentum: fma(.05, g - m, m)
+        want = torch.lerp(want, g[i].cpu(), .05)
+        assert torch.equal(results[0][1][i].cpu(), want), i
+
+
 @pytest.mark.parametrize("alpha", [1 + 2 ** -8, 1 + 3 * 2 ** -8, 1 / 3, -0.7, 2.0 ** -140, 7.5e37])
 def test_gemm_output_rounding_is_round_to_nearest_even(alpha):
     """C = alpha * I Q^T is one fp32 product alpha * q rounded once to bf16.  With q a
