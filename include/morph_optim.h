@@ -255,6 +255,35 @@ int morph_nonfinite_or_close(const void* const* grads, const int64_t* numels, in
                              int dtype, morph_step_state* d_state, int slot, int64_t* d_clocks,
                              const int32_t* d_prev_clock_list, int n_prev, void* stream);
 
+/* ---- A group of many tensors in one launch ---------------------------------
+ * morph_adamw_multi_dev carries its descriptors in the kernel arguments, 48 tensors to a
+ * launch.  For a group of hundreds of small tensors the caller may keep them in device
+ * memory instead: fill a host image once (pointers, sizes, constant sets, clocks; the
+ * gradients are not part of it), copy it to the device, and pass it with the same
+ * tensors[] (which carry the step's gradients) to the two calls below, 400 tensors to a
+ * launch.  The image is valid while numel, param, exp_avg, exp_avg_sq, out, hp_index,
+ * clock_index, their order, grad_dtype and whether there is an export stay as they were.
+ * Limits: 2^30 elements per tensor, 8 constant sets (MORPH_ERANGE).  Same references as
+ * morph_adamw_multi_dev and morph_nonfinite_or_close.
+ */
+
+/* Bytes of the table (a multiple of 4), or a negative status. */
+int64_t morph_adamw_table_bytes(const morph_adamw_tensor* tensors, int count, int grad_dtype);
+/* Fills the host image at host_table (8-byte aligned). */
+int morph_adamw_table_fill(const morph_adamw_tensor* tensors, int count, int grad_dtype,
+                           int out_dtype, void* host_table, int64_t bytes);
+/* morph_adamw_multi_dev over the table at d_table (64-byte aligned), same results. */
+int morph_adamw_table_dev(const void* d_table, const morph_adamw_tensor* tensors, int count,
+                          int grad_dtype, int out_dtype, const morph_adamw_hp* hps,
+                          const morph_adamw_sched* scheds, int n_hp, const int64_t* d_clocks,
+                          const morph_step_state* d_state, int slot, void* start_event,
+                          void* stop_event, void* stream);
+/* The detector over the table's gradients into d_state->found_inf[slot]; close != 0: with
+ * the previous step's close, as morph_nonfinite_or_close. */
+int morph_nonfinite_table(const void* d_table, const morph_adamw_tensor* tensors, int count,
+                          int grad_dtype, morph_step_state* d_state, int slot, int64_t* d_clocks,
+                          const int32_t* d_prev_clock_list, int n_prev, int close, void* stream);
+
 /* ---- Stage-gradient accumulation ------------------------------------------
  * Replaces the reference's per-micro-batch
  *   destination.add_(g.detach().float() / loss_scale)

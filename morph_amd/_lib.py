@@ -15,6 +15,8 @@ import torch  # noqa: F401  (must load the HIP runtime before the library)
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libmorph_optim.so"
 ABI_VERSION = 9
+ADAMW_LAUNCH_TENSORS = 48  # tensors of one morph_adamw_multi launch
+ADAMW_TABLE_SETS, ADAMW_TABLE_NUMEL = 8, 1 << 30  # limits of morph_adamw_table_dev
 
 DTYPE_NONE, DTYPE_F32, DTYPE_F16, DTYPE_BF16 = -1, 0, 1, 2
 HP_DIVIDE_SCALE, HP_APPLY_CLIP, HP_APPLY_DECAY, HP_LERP_LARGE = 1, 2, 4, 8
@@ -23,7 +25,8 @@ HP_DIVIDE_SCALE, HP_APPLY_CLIP, HP_APPLY_DECAY, HP_LERP_LARGE = 1, 2, 4, 8
 EXPORTS = (
     "morph_abi_version", "morph_strerror", "morph_flag_clear", "morph_nonfinite_or",
     "morph_nonfinite_or_multi", "morph_adamw_fused", "morph_adamw_multi",
-    "morph_adamw_multi_dev", "morph_step_end", "morph_nonfinite_or_close",
+    "morph_adamw_multi_dev", "morph_adamw_table_bytes", "morph_adamw_table_fill",
+    "morph_adamw_table_dev", "morph_nonfinite_table", "morph_step_end", "morph_nonfinite_or_close",
     "morph_grad_partials", "morph_grad_accumulate", "morph_grad_accumulate_final_noalloc",
     "morph_sumsq_total", "morph_convert_f32", "morph_fp8_pack", "morph_fp8_unpack",
     "morph_gemm_nt_bf16",
@@ -130,6 +133,13 @@ def _load():
         "morph_adamw_multi_dev": ([ctypes.POINTER(AdamwTensor), i32, i32, i32,
                                    ctypes.POINTER(AdamwHP), ctypes.POINTER(AdamwSched), i32,
                                    vp, vp, i32, vp, vp, vp], i32),
+        "morph_adamw_table_bytes": ([ctypes.POINTER(AdamwTensor), i32, i32], i64),
+        "morph_adamw_table_fill": ([ctypes.POINTER(AdamwTensor), i32, i32, i32, vp, i64], i32),
+        "morph_adamw_table_dev": ([vp, ctypes.POINTER(AdamwTensor), i32, i32, i32,
+                                   ctypes.POINTER(AdamwHP), ctypes.POINTER(AdamwSched), i32,
+                                   vp, vp, i32, vp, vp, vp], i32),
+        "morph_nonfinite_table": ([vp, ctypes.POINTER(AdamwTensor), i32, i32, vp, i32, vp, vp,
+                                   i32, i32, vp], i32),
         "morph_step_end": ([vp, vp, vp, i32, i32, vp], i32),
         "morph_nonfinite_or_close": ([vp, vp, i32, i32, vp, i32, vp, vp, i32, vp], i32),
         "morph_grad_partials": ([ctypes.POINTER(AccumTensor), i32], i64),

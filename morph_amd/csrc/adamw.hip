@@ -36,6 +36,7 @@
 // loop can enqueue steps without waiting for the previous outcome.
 #include <hip/hip_ext.h>
 
+#include "adamw_table.h"
 #include "common.h"
 
 #ifndef MORPH_ADAMW_UNROLL
@@ -249,8 +250,8 @@ __device__ __forceinline__ void chunk_scalar(const TensorArg& T, const morph_ada
 // The step's constants for this workgroup's tensor, or false when the step
 // must leave memory untouched (overflow flagged, fatal state, or a clock
 // outside the tables).
-template <bool kDev>
-__device__ __forceinline__ bool control(const LaunchArgs& a, const TensorArg& T,
+template <bool kDev, typename Args>
+__device__ __forceinline__ bool control(const Args& a, const TensorArg& T,
                                         const uint32_t* skip, morph_adamw_hp& hp) {
   hp = a.hp[T.hp];
   if constexpr (kDev) {
@@ -272,11 +273,10 @@ __device__ __forceinline__ bool control(const LaunchArgs& a, const TensorArg& T,
   return true;
 }
 
-template <typename GT, typename OT, bool kDev>
-__global__ __launch_bounds__(kBlock) void adamw_multi_kernel(const LaunchArgs a,
-                                                             const uint32_t* __restrict__ skip) {
-  const int b = a.reverse ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
-  const TensorArg& T = a.t[segment_of(a.t, a.count, b)];
+// Block b of tensor T.
+template <typename GT, typename OT, bool kDev, typename Args>
+__device__ __forceinline__ void run_block(const Args& a, const TensorArg& T, int b,
+                                          const uint32_t* skip) {
   const int64_t base = (int64_t)(b - T.first_block) * kPerBlock;
   morph_adamw_hp hp;
   if (T.vector_ok && base + kPerBlock <= T.n) {
@@ -290,6 +290,41 @@ __global__ __launch_bounds__(kBlock) void adamw_multi_kernel(const LaunchArgs a,
     if (!control<kDev>(a, T, skip, hp)) return;
     chunk_scalar<GT, OT>(T, hp, base, base + kPerBlock < T.n ? base + kPerBlock : T.n);
   }
+}
+
+template <typename GT, typename OT, bool kDev>
+__global__ __launch_bounds__(kBlock) void adamw_multi_kernel(const LaunchArgs a,
+                                                             const uint32_t* __restrict__ skip) {
+  const int b = a.reverse ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
+  run_block<GT, OT, kDev>(a, a.t[segment_of(a.t, a.count, b)], b, skip);
+}
+
+// Many tensors in one launch (adamw_table.h): the descriptors lie in device memory, the
+// gradients' addresses in the kernel arguments (bit 0: the tensor takes 4-byte accesses).
+struct TableArgs {
+  uint64_t grad[kTableRefs];
+  morph_adamw_hp hp[kMaxHp];
+  morph_adamw_sched sched[kMaxHp];
+  const int64_t* clocks;
+  const morph_step_state* state;
+  int32_t first_row, first_block;
+  int32_t reverse;
+};
+static_assert(sizeof(TableArgs) + 64 <= kMaxKernargBytes, "launch table fits the kernel arguments");
+
+template <typename GT, typename OT>
+__global__ __launch_bounds__(kBlock) void adamw_table_kernel(const TableArgs a,
+                                                             const TableRow* __restrict__ rows,
+                                                             const int32_t* __restrict__ map,
+                                                             const uint32_t* __restrict__ skip) {
+  const int b = a.first_block +
+                (a.reverse ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
+  const int row = __builtin_amdgcn_readfirstlane(map[b]);
+  const TableRow& R = rows[row];
+  const uint64_t g = a.grad[row - a.first_row];
+  const TensorArg T{reinterpret_cast<const void*>(g & ~uint64_t(1)), R.p, R.m, R.v, R.out, R.n,
+                    R.hp, R.first_block, (int32_t)(~g & 1), R.clock};
+  run_block<GT, OT, true>(a, T, b, skip);
 }
 
 // Events (nullable) are stamped by the dispatch itself (hipExtLaunchKernel):
@@ -351,6 +386,13 @@ int dtype_bytes(int dtype) {
 }
 
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
+
+// 4 elements per access on every stream of the tensor.
+bool vector_ok(const void* p, const void* m, const void* v, const void* grad, int gb,
+               const void* out, int ob) {
+  return aligned(p, 16) && aligned(m, 16) && aligned(v, 16) && aligned(grad, 4 * gb) &&
+         (out == nullptr || aligned(out, 4 * ob));
+}
 
 // Validates everything, then splits the tensor list into launches of at most
 // kMaxTensors segments and kMaxHp constant sets.  `scheds`, `clocks` and
@@ -431,8 +473,7 @@ int enqueue(const morph_adamw_tensor* tensors, int count, int grad_dtype, int ou
       d.n = n;
       d.hp = local;
       d.first_block = blocks;
-      d.vector_ok = aligned(d.p, 16) && aligned(d.m, 16) && aligned(d.v, 16) &&
-                    aligned(d.grad, 4 * gb) && (d.out == nullptr || aligned(d.out, 4 * ob));
+      d.vector_ok = vector_ok(d.p, d.m, d.v, d.grad, gb, d.out, ob);
       d.clock = dev ? t.clock_index : 0;
       blocks += (int)((n + kPerBlock - 1) / kPerBlock);
       grad_bytes += n * gb;
@@ -445,6 +486,158 @@ int enqueue(const morph_adamw_tensor* tensors, int count, int grad_dtype, int ou
 }  // namespace morph
 
 using namespace morph;
+
+// ---- The descriptor table (adamw_table.h) -----------------------------------
+namespace {
+
+// Blocks of AdamW and of the detector that each tensor owns, in table order.
+struct TableShape {
+  int64_t blocks = 0, det_blocks = 0;
+};
+
+int table_shape(const morph_adamw_tensor* tensors, int count, int grad_dtype, TableShape* out) {
+  const int gb = dtype_bytes(grad_dtype);
+  if (gb == 0) return MORPH_EDTYPE;
+  if (count < 0 || (count > 0 && tensors == nullptr)) return MORPH_EINVAL;
+  TableShape t;
+  for (int i = 0; i < count; ++i) {
+    const int64_t n = tensors[i].numel;
+    if (n < 0) return MORPH_EINVAL;
+    if (n > kMaxSegment) return MORPH_ERANGE;
+    t.blocks += (n + kPerBlock - 1) / kPerBlock;
+    t.det_blocks += (n * gb + kDetectorBytes - 1) / kDetectorBytes;
+  }
+  if (t.blocks > INT32_MAX - 1 || t.det_blocks > INT32_MAX - 1) return MORPH_ERANGE;
+  *out = t;
+  return MORPH_OK;
+}
+
+int64_t table_bytes(int count, const TableShape& t) {
+  return (int64_t)count * (int64_t)sizeof(TableRow) + 4 * (t.blocks + t.det_blocks);
+}
+
+template <typename GT, typename OT>
+int launch_table(const TableArgs& a, const void* d_table, int count, int blocks,
+                 const uint32_t* skip, hipStream_t s, Stamps ev) {
+  const TableRow* rows = static_cast<const TableRow*>(d_table);
+  const int32_t* map = reinterpret_cast<const int32_t*>(rows + count);
+  if (ev.e0 == nullptr && ev.e1 == nullptr)
+    hipLaunchKernelGGL((adamw_table_kernel<GT, OT>), dim3(blocks), dim3(kBlock), kOccupancyLds, s,
+                       a, rows, map, skip);
+  else
+    hipExtLaunchKernelGGL((adamw_table_kernel<GT, OT>), dim3(blocks), dim3(kBlock), kOccupancyLds,
+                          s, ev.e0, ev.e1, 0u, a, rows, map, skip);
+  return launch_status();
+}
+
+template <typename GT>
+int launch_table_out(int out_dtype, const TableArgs& a, const void* d_table, int count, int blocks,
+                     const uint32_t* skip, hipStream_t s, Stamps ev) {
+  switch (out_dtype) {
+    case MORPH_DTYPE_NONE: return launch_table<GT, NoOut>(a, d_table, count, blocks, skip, s, ev);
+    case MORPH_DTYPE_F32: return launch_table<GT, F32>(a, d_table, count, blocks, skip, s, ev);
+    case MORPH_DTYPE_F16: return launch_table<GT, F16>(a, d_table, count, blocks, skip, s, ev);
+    case MORPH_DTYPE_BF16: return launch_table<GT, BF16>(a, d_table, count, blocks, skip, s, ev);
+    default: return MORPH_EDTYPE;
+  }
+}
+
+}  // namespace
+
+extern "C" int64_t morph_adamw_table_bytes(const morph_adamw_tensor* tensors, int count,
+                                           int grad_dtype) {
+  TableShape t;
+  const int rc = table_shape(tensors, count, grad_dtype, &t);
+  return rc != MORPH_OK ? rc : table_bytes(count, t);
+}
+
+extern "C" int morph_adamw_table_fill(const morph_adamw_tensor* tensors, int count, int grad_dtype,
+                                      int out_dtype, void* host_table, int64_t bytes) {
+  TableShape t;
+  const int rc = table_shape(tensors, count, grad_dtype, &t);
+  if (rc != MORPH_OK) return rc;
+  if (count > 0 && host_table == nullptr) return MORPH_EINVAL;
+  if (bytes < table_bytes(count, t)) return MORPH_EWORKSPACE;
+  const int gb = dtype_bytes(grad_dtype);
+  TableRow* rows = static_cast<TableRow*>(host_table);
+  int32_t* map = reinterpret_cast<int32_t*>(rows + count);
+  int32_t* det = map + t.blocks;
+  int32_t block = 0, det_block = 0;
+  for (int i = 0; i < count; ++i) {
+    const morph_adamw_tensor& x = tensors[i];
+    if (x.numel > 0 && (x.param == nullptr || x.exp_avg == nullptr || x.exp_avg_sq == nullptr))
+      return MORPH_EINVAL;
+    if (x.hp_index < 0 || x.hp_index >= kMaxHp || x.clock_index < 0) return MORPH_EINVAL;
+    rows[i] = TableRow{x.param, x.exp_avg, x.exp_avg_sq,
+                       out_dtype == MORPH_DTYPE_NONE ? nullptr : x.out, x.numel, x.hp_index,
+                       x.clock_index, block, det_block, {0, 0}};
+    for (int64_t k = (x.numel + kPerBlock - 1) / kPerBlock; k > 0; --k) map[block++] = i;
+    for (int64_t k = (x.numel * gb + kDetectorBytes - 1) / kDetectorBytes; k > 0; --k)
+      det[det_block++] = i;
+  }
+  return MORPH_OK;
+}
+
+extern "C" int morph_adamw_table_dev(const void* d_table, const morph_adamw_tensor* tensors,
+                                     int count, int grad_dtype, int out_dtype,
+                                     const morph_adamw_hp* hps, const morph_adamw_sched* scheds,
+                                     int n_hp, const int64_t* d_clocks,
+                                     const morph_step_state* d_state, int slot, void* start_event,
+                                     void* stop_event, void* stream) {
+  TableShape shape;
+  int rc = table_shape(tensors, count, grad_dtype, &shape);
+  if (rc != MORPH_OK) return rc;
+  if (d_state == nullptr || (slot != 0 && slot != 1) || n_hp < 0) return MORPH_EINVAL;
+  if (n_hp > kMaxHp) return MORPH_ERANGE;
+  if (count > 0 && (d_table == nullptr || hps == nullptr || scheds == nullptr || d_clocks == nullptr))
+    return MORPH_EINVAL;
+  if (out_dtype != MORPH_DTYPE_NONE && dtype_bytes(out_dtype) == 0) return MORPH_EDTYPE;
+  const int gb = dtype_bytes(grad_dtype);
+  const int ob = out_dtype == MORPH_DTYPE_NONE ? 0 : dtype_bytes(out_dtype);
+  TableArgs a;
+  for (int k = 0; k < n_hp; ++k) {
+    if (scheds[k].table_len < 1 || scheds[k].bias_correction1 == nullptr ||
+        scheds[k].bias_correction2_sqrt == nullptr)
+      return MORPH_EINVAL;
+    a.hp[k] = hps[k];
+    a.sched[k] = scheds[k];
+  }
+  for (int i = 0; i < count; ++i)
+    if (tensors[i].hp_index < 0 || tensors[i].hp_index >= n_hp ||
+        (tensors[i].numel > 0 && tensors[i].grad == nullptr))
+      return MORPH_EINVAL;
+  a.clocks = d_clocks;
+  a.state = d_state;
+  hipStream_t s = as_stream(stream);
+  int64_t block = 0;
+  for (int r0 = 0; r0 < count; r0 += kTableRefs) {
+    const int r1 = count - r0 < kTableRefs ? count : r0 + kTableRefs;
+    a.first_row = r0;
+    a.first_block = (int32_t)block;
+    int64_t grad_bytes = 0, blocks = 0;
+    for (int i = r0; i < r1; ++i) {
+      const morph_adamw_tensor& x = tensors[i];
+      const bool vec = vector_ok(x.param, x.exp_avg, x.exp_avg_sq, x.grad, gb,
+                                 ob != 0 ? x.out : nullptr, ob);
+      a.grad[i - r0] = reinterpret_cast<uintptr_t>(x.grad) | (vec ? 0u : 1u);
+      blocks += (x.numel + kPerBlock - 1) / kPerBlock;
+      grad_bytes += x.numel * gb;
+    }
+    a.reverse = grad_bytes > kReverseAboveBytes ? 1 : 0;
+    const Stamps ev{r0 == 0 ? static_cast<hipEvent_t>(start_event) : nullptr,
+                    r1 == count ? static_cast<hipEvent_t>(stop_event) : nullptr};
+    block += blocks;
+    if (blocks == 0) continue;
+    const uint32_t* skip = &d_state->found_inf[slot];
+    switch (grad_dtype) {
+      case MORPH_DTYPE_F32: rc = launch_table_out<F32>(out_dtype, a, d_table, count, (int)blocks, skip, s, ev); break;
+      case MORPH_DTYPE_F16: rc = launch_table_out<F16>(out_dtype, a, d_table, count, (int)blocks, skip, s, ev); break;
+      default: rc = launch_table_out<BF16>(out_dtype, a, d_table, count, (int)blocks, skip, s, ev); break;
+    }
+    if (rc != MORPH_OK) return rc;
+  }
+  return MORPH_OK;
+}
 
 extern "C" int morph_adamw_multi(const morph_adamw_tensor* tensors, int count, int grad_dtype,
                                  int out_dtype, const morph_adamw_hp* hps, int n_hp,

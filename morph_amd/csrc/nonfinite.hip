@@ -16,6 +16,7 @@
 // morph_nonfinite_or_close adds one workgroup (the first) that closes the
 // previous optimizer step (close_step), which saves that close its own launch.  It reads and clears only the other step's flag word, so the
 // detector workgroups and the close may run in any order.
+#include "adamw_table.h"
 #include "common.h"
 #include "step_close.h"
 
@@ -35,6 +36,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kUnroll = MORPH_NONFINITE_UNROLL;
 constexpr int kBytesPerBlock = kBlock * 16 * kUnroll;
+static_assert(kBytesPerBlock == kDetectorBytes, "the table's detector blocks");
 constexpr int kMaxTensors = 160;
 constexpr int64_t kMaxSegmentBytes = int64_t(1) << 32;
 
@@ -75,12 +77,36 @@ struct CloseArgs {
   int32_t slot;
 };
 
+// Block `block` of the n elements at g.
+template <typename GT>
+__device__ __forceinline__ void scan_block(const void* g, int64_t n, bool vector_ok, int block,
+                                           uint32_t* flag) {
+  constexpr int kElemBytes = Fmt<GT>::bytes;
+  constexpr int kPerBlock = kBytesPerBlock / kElemBytes;
+  const int64_t base = (int64_t)block * kPerBlock;
+  bool bad = false;
+  if (vector_ok && base + kPerBlock <= n) {
+    const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const char*>(g) +
+                                                    base * kElemBytes);
+    u32x4 w[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      w[u] = load_stream<MORPH_NONFINITE_NT != 0>(p + u * kBlock + threadIdx.x);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      bad |= word_nonfinite<GT>(w[u].x) | word_nonfinite<GT>(w[u].y) |
+             word_nonfinite<GT>(w[u].z) | word_nonfinite<GT>(w[u].w);
+  } else {
+    const int64_t end = base + kPerBlock < n ? base + kPerBlock : n;
+    for (int64_t i = base + threadIdx.x; i < end; i += kBlock) bad |= elem_nonfinite<GT>(g, i);
+  }
+  if (__any(bad) && (threadIdx.x & 63) == 0) *reinterpret_cast<volatile uint32_t*>(flag) = 1u;
+}
+
 template <typename GT, bool kClose>
 __global__ __launch_bounds__(kBlock) void nonfinite_kernel(const LaunchArgs a,
                                                            uint32_t* __restrict__ flag,
                                                            const CloseArgs c) {
-  constexpr int kElemBytes = Fmt<GT>::bytes;
-  constexpr int kPerBlock = kBytesPerBlock / kElemBytes;
   int b = blockIdx.x;
   if constexpr (kClose) {
     // Workgroup 0 closes the previous step: dispatched first, its chain of
@@ -92,24 +118,47 @@ __global__ __launch_bounds__(kBlock) void nonfinite_kernel(const LaunchArgs a,
     b -= 1;
   }
   const TensorArg& T = a.t[segment_of(a.t, a.count, b)];
-  const int64_t base = (int64_t)(b - T.first_block) * kPerBlock;
-  bool bad = false;
-  if (T.vector_ok && base + kPerBlock <= T.n) {
-    const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const char*>(T.g) +
-                                                    base * kElemBytes);
-    u32x4 w[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      w[u] = load_stream<MORPH_NONFINITE_NT != 0>(p + u * kBlock + threadIdx.x);
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      bad |= word_nonfinite<GT>(w[u].x) | word_nonfinite<GT>(w[u].y) |
-             word_nonfinite<GT>(w[u].z) | word_nonfinite<GT>(w[u].w);
-  } else {
-    const int64_t end = base + kPerBlock < T.n ? base + kPerBlock : T.n;
-    for (int64_t i = base + threadIdx.x; i < end; i += kBlock) bad |= elem_nonfinite<GT>(T.g, i);
+  scan_block<GT>(T.g, T.n, T.vector_ok != 0, b - T.first_block, flag);
+}
+
+// Many tensors in one launch (adamw_table.h): sizes and the block map lie in device
+// memory, the gradients' addresses in the kernel arguments (bit 0: not on 16 bytes).
+struct TableArgs {
+  uint64_t grad[kTableRefs];
+  int32_t first_row, first_block;
+};
+static_assert(sizeof(TableArgs) + sizeof(CloseArgs) + 64 <= kMaxKernargBytes,
+              "launch table fits the kernel arguments");
+
+template <typename GT, bool kClose>
+__global__ __launch_bounds__(kBlock) void nonfinite_table_kernel(
+    const TableArgs a, const TableRow* __restrict__ rows, const int32_t* __restrict__ map,
+    uint32_t* __restrict__ flag, const CloseArgs c) {
+  int b = blockIdx.x;
+  if constexpr (kClose) {  // workgroup 0, as in nonfinite_kernel
+    if (b == 0) {
+      close_step(c.state, c.clocks, c.list, c.n, c.slot, kBlock);
+      return;
+    }
+    b -= 1;
   }
-  if (__any(bad) && (threadIdx.x & 63) == 0) *reinterpret_cast<volatile uint32_t*>(flag) = 1u;
+  b += a.first_block;
+  const int row = __builtin_amdgcn_readfirstlane(map[b]);
+  const uint64_t g = a.grad[row - a.first_row];
+  scan_block<GT>(reinterpret_cast<const void*>(g & ~uint64_t(1)), rows[row].n, (g & 1) == 0,
+                 b - rows[row].det_first, flag);
+}
+template <typename GT>
+int launch_table(const TableArgs& a, const void* d_table, const int32_t* map, int blocks,
+                 uint32_t* flag, const CloseArgs* close, hipStream_t s) {
+  const TableRow* rows = static_cast<const TableRow*>(d_table);
+  if (close != nullptr)
+    hipLaunchKernelGGL((nonfinite_table_kernel<GT, true>), dim3(blocks + 1), dim3(kBlock), 0, s, a,
+                       rows, map, flag, *close);
+  else
+    hipLaunchKernelGGL((nonfinite_table_kernel<GT, false>), dim3(blocks), dim3(kBlock), 0, s, a,
+                       rows, map, flag, CloseArgs{});
+  return launch_status();
 }
 
 template <typename GT>
@@ -212,6 +261,59 @@ extern "C" int morph_nonfinite_or_close(const void* const* grads, const int64_t*
   const CloseArgs close{d_state, d_clocks, d_prev_clock_list, n_prev, slot ^ 1};
   return nonfinite_impl(grads, numels, count, dtype, &d_state->found_inf[slot], &close,
                         as_stream(stream));
+}
+
+extern "C" int morph_nonfinite_table(const void* d_table, const morph_adamw_tensor* tensors,
+                                     int count, int grad_dtype, morph_step_state* d_state, int slot,
+                                     int64_t* d_clocks, const int32_t* d_prev_clock_list,
+                                     int n_prev, int close, void* stream) {
+  const int64_t bytes = morph_adamw_table_bytes(tensors, count, grad_dtype);
+  if (bytes < 0) return (int)bytes;
+  if (d_state == nullptr || (slot != 0 && slot != 1) || n_prev < 0 ||
+      (count > 0 && d_table == nullptr) ||
+      (close != 0 && n_prev > 0 && (d_clocks == nullptr || d_prev_clock_list == nullptr)))
+    return MORPH_EINVAL;
+  int eb;
+  switch (grad_dtype) {
+    case MORPH_DTYPE_F32: eb = 4; break;
+    default: eb = 2; break;
+  }
+  int64_t total = 0;
+  for (int i = 0; i < count; ++i) {
+    if (tensors[i].numel > 0 && tensors[i].grad == nullptr) return MORPH_EINVAL;
+    total += (tensors[i].numel * eb + kDetectorBytes - 1) / kDetectorBytes;
+  }
+  // the detector's map is the table's last part
+  const int32_t* map = reinterpret_cast<const int32_t*>(static_cast<const char*>(d_table) + bytes -
+                                                        4 * total);
+  const CloseArgs ca{d_state, d_clocks, d_prev_clock_list, n_prev, slot ^ 1};
+  const CloseArgs* pending = close != 0 ? &ca : nullptr;
+  uint32_t* flag = &d_state->found_inf[slot];
+  hipStream_t s = as_stream(stream);
+  TableArgs a;
+  int64_t block = 0;
+  for (int r0 = 0; r0 < count || pending != nullptr; r0 += kTableRefs) {
+    const int r1 = count - r0 < kTableRefs ? count : r0 + kTableRefs;
+    a.first_row = r0;
+    a.first_block = (int32_t)block;
+    int64_t blocks = 0;
+    for (int i = r0; i < r1; ++i) {
+      const uintptr_t g = reinterpret_cast<uintptr_t>(tensors[i].grad);
+      a.grad[i - r0] = g % 16 == 0 ? g : g | 1u;
+      blocks += (tensors[i].numel * eb + kDetectorBytes - 1) / kDetectorBytes;
+    }
+    block += blocks;
+    if (blocks == 0 && pending == nullptr) continue;
+    int rc;
+    switch (grad_dtype) {
+      case MORPH_DTYPE_F32: rc = launch_table<F32>(a, d_table, map, (int)blocks, flag, pending, s); break;
+      case MORPH_DTYPE_F16: rc = launch_table<F16>(a, d_table, map, (int)blocks, flag, pending, s); break;
+      default: rc = launch_table<BF16>(a, d_table, map, (int)blocks, flag, pending, s); break;
+    }
+    if (rc != MORPH_OK) return rc;
+    pending = nullptr;
+  }
+  return MORPH_OK;
 }
 
 extern "C" int morph_nonfinite_or(const void* grad, int dtype, int64_t n, uint32_t* d_flag,

@@ -107,9 +107,54 @@ class AdamwBatch:
             d.clock_index = clock_index[i]
             keep.append((p, m, v, g, o))
         self._keep = keep  # the tensors must outlive the descriptors
+        self._table = self._device_table() if n > _lib.ADAMW_LAUNCH_TENSORS else None
         self._grad_dtype = grads[0].dtype if n else None
         self._numels = [p.numel() for p in params]
         self._device = params[0].device if n else None
+
+    def _device_table(self):
+        """The descriptors in device memory (morph_adamw_table_fill), for the one-launch forms
+        of groups with more tensors than the kernel arguments hold; None outside its limits."""
+        if (self.n_hp > _lib.ADAMW_TABLE_SETS
+                or any(d.numel > _lib.ADAMW_TABLE_NUMEL for d in self.array)
+                or any(d.clock_index < 0 for d in self.array)):
+            return None
+        L = lib()
+        nbytes = L.morph_adamw_table_bytes(self.array, self.count, self.grad_dtype)
+        check(nbytes if nbytes < 0 else 0)
+        host = torch.empty(nbytes, dtype=torch.uint8)
+        check(L.morph_adamw_table_fill(self.array, self.count, self.grad_dtype, self.out_dtype,
+                                       _ptr(host), nbytes))
+        self._table_stream = torch.cuda.current_stream(self._keep[0][0].device)
+        return host.to(self._keep[0][0].device)
+
+    def _use_table(self, stream):
+        """The table, kept for work enqueued on another stream than the one that was current
+        when it was allocated."""
+        if stream is not None and stream != self._table_stream:
+            self._table.record_stream(stream)
+        return _ptr(self._table)
+
+    def detect(self, grads, state, slot, clocks, prev_clock_list=None, stream=None):
+        """One detector pass over the gradients that the descriptors point at (`grads`, checked
+        again) into found_inf[slot] of `state`, with the previous step's close when
+        prev_clock_list is given (nonfinite_or_close)."""
+        if self._table is None:
+            if prev_clock_list is not None:
+                nonfinite_or_close(grads, state, slot, clocks, prev_clock_list, stream)
+            else:
+                nonfinite_or(grads, state.data_ptr() + _lib.StepState.found_inf.offset + 4 * slot,
+                             stream)
+            return
+        for i, g in enumerate(grads):
+            require_device_tensor(g, f"grads[{i}]")
+        close = prev_clock_list is not None
+        if close:
+            _check_close_args(state, clocks, prev_clock_list)
+        check(lib().morph_nonfinite_table(
+            self._use_table(stream), self.array, self.count, self.grad_dtype, _ptr(state), slot,
+            _ptr(clocks) if close else None, _ptr(prev_clock_list) if close else None,
+            prev_clock_list.numel() if close else 0, int(close), stream_handle(stream)))
 
     def rebind_grads(self, grads):
         """Point the descriptors at new gradient tensors of the same sizes and dtype.
@@ -165,6 +210,12 @@ class AdamwBatch:
         harr = (_lib.AdamwHP * len(hps))(*hps)
         sarr = (_lib.AdamwSched * len(scheds))(*scheds)
         e0, e1 = _event_handles(events)
+        if self._table is not None and len(hps) <= _lib.ADAMW_TABLE_SETS:
+            check(lib().morph_adamw_table_dev(self._use_table(stream), self.array, self.count,
+                                              self.grad_dtype, self.out_dtype, harr, sarr,
+                                              len(hps), _ptr(clocks), _ptr(state), slot, e0, e1,
+                                              stream_handle(stream)))
+            return
         check(lib().morph_adamw_multi_dev(self.array, self.count, self.grad_dtype,
                                           self.out_dtype, harr, sarr, len(hps), _ptr(clocks),
                                           _ptr(state), slot, e0, e1, stream_handle(stream)))

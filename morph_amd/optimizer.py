@@ -429,12 +429,10 @@ class FusedAdamW:
             s.wait_stream(prev)
         if checked:
             self._flush_close()
-        elif self._pending is not None:
-            kernels.nonfinite_or_close([grads[i] for i in present], ctl.state, slot, ctl.clocks,
-                                       self._pending[1], s)
-            self._pending = None
         else:
-            kernels.nonfinite_or([grads[i] for i in present], ctl.found_inf_ptr(slot), s)
+            prev = self._pending[1] if self._pending is not None else None
+            batch.detect([grads[i] for i in present], ctl.state, slot, ctl.clocks, prev, s)
+            self._pending = None
         if pipeline:
             flat = self._flat()
             groups = sorted({flat[i][0] for i in present})

@@ -502,6 +502,51 @@ def test_fused_close_with_a_detector_over_several_launches():
         assert a.state[p]["step"] == b.state[q]["step"] == 6
 
 
+@pytest.mark.parametrize("dtype,export,count", [(torch.float32, None, 49), (torch.float16, torch.float16, 401),
+                                                (torch.bfloat16, torch.bfloat16, 830)])
+def test_descriptor_table_equals_kernel_argument_launches(monkeypatch, dtype, export, count):
+    """More than 48 tensors run over the descriptor table in device memory (400 gradients a
+    launch), the same bytes as the launches whose descriptors are kernel arguments: sizes at
+    the edges of the AdamW and detector blocks, empty ones, views off 16 bytes, two constant
+    sets, new gradient buffers, a non-finite value in the first and the last tensor."""
+    from morph_amd import kernels
+    edges = [0, 1, 3, 255, 256, 257, 4095, 4096, 4097, 8191, 8192, 8193, 20000]
+    gen = torch.Generator().manual_seed(count)
+    sizes = [edges[i % len(edges)] if i % 3 else int(torch.randint(1, 700, (1,), generator=gen))
+             for i in range(count)]
+    sizes[0], sizes[-1] = 300, 8193
+    place = lambda t, i: torch.cat([torch.zeros(i % 4, dtype=t.dtype), t]).to(DEV)[i % 4:]  # noqa: E731
+    masters = [torch.randn(n, generator=gen) * .02 for n in sizes]
+    steps = [[(torch.randn(n, generator=gen) * 1e-3 * 64).to(dtype) for n in sizes] for _ in range(4)]
+    steps[1][0][299] = float("nan")
+    steps[2][-1][8192] = float("inf")
+    runs = []
+    for table in (True, False):
+        if not table:
+            monkeypatch.setattr(kernels.AdamwBatch, "_device_table", lambda self: None)
+        ps = [place(m, i) for i, m in enumerate(masters)]
+        opt = FusedAdamW([dict(params=ps[:7]), dict(params=ps[7:], lr=2e-3, weight_decay=0.0)], lr=1e-3,
+                         loss_scale=DynamicLossScale(64.0), export_dtype=export)
+        outs = []
+        for k, gs in enumerate(steps):
+            gs = [place(g, i if k else 0) for i, g in enumerate(gs)]
+            assert (opt._cache is None) or (opt._cache[0]._table is not None) == table
+            opt.step(gs)
+            outs.append([p.clone() for p in ps])
+        opt.resolve()
+        outs.append([opt.state[p][k] for p in ps for k in ("exp_avg", "exp_avg_sq")] + opt.exports)
+        runs.append((opt, outs))
+    (a, oa), (b, ob) = runs
+    assert a.skipped_steps == b.skipped_steps == 2 and a.applied_steps == b.applied_steps == 2
+    for step, (xs, ys) in enumerate(zip(oa, ob)):
+        for i, (x, y) in enumerate(zip(xs, ys)):
+            assert torch.equal(x, y), (step, i)
+    assert not torch.equal(oa[0][0], oa[3][0]) and torch.equal(oa[0][0], oa[2][0])
+    strided = torch.zeros(2 * sizes[0], dtype=dtype, device=DEV)[::2]
+    with pytest.raises(ValueError, match="contiguous"):
+        a.step([strided] + [torch.zeros(n, dtype=dtype, device=DEV) for n in sizes[1:]])
+
+
 @pytest.mark.parametrize("count,size", [(1, 1 << 24), (200, 1 << 16)], ids=["one", "split"])
 def test_dispatch_timer_stamps_the_adamw_launches(count, size):
     """Events stamped by the AdamW dispatch itself (hipExtLaunchKernel) time the pass: each
