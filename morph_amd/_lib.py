@@ -8,12 +8,14 @@ pointers are valid in both.  There is no fallback: when the library is missing
 every entry point raises.
 """
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
 import torch  # noqa: F401  (must load the HIP runtime before the library)
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libmorph_optim.so"
+HOSTPATH_PATH = LIB_PATH.with_name("_hostpath.so")
 ABI_VERSION = 9
 ADAMW_LAUNCH_TENSORS = 48  # tensors of one morph_adamw_multi launch
 ADAMW_TABLE_SETS, ADAMW_TABLE_NUMEL = 8, 1 << 30  # limits of morph_adamw_table_dev
@@ -179,6 +181,30 @@ def _load():
     if version != ABI_VERSION:
         raise ImportError(f"{LIB_PATH} has ABI {version}, expected {ABI_VERSION}")
     _lib = handle
+
+
+_hostpath = None
+
+
+def hostpath():
+    """The host extension (hostpath.cpp), loaded once; raises if it has not been built."""
+    global _hostpath
+    if _hostpath is None:
+        with _load_lock:
+            if _hostpath is None:
+                if not HOSTPATH_PATH.exists():
+                    raise ImportError(f"{HOSTPATH_PATH} is missing: build it first "
+                                      "(python -m morph_amd.build)")
+                spec = importlib.util.spec_from_file_location("_hostpath", HOSTPATH_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _hostpath = module
+    return _hostpath
+
+
+def entry_address(name):
+    """The address of one of the library's entry points."""
+    return ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
 
 
 def check(status):

@@ -1,4 +1,4 @@
-"""Build libmorph_optim.so for gfx950 in-tree (python -m morph_amd.build).
+"""Build libmorph_optim.so for gfx950 and the host extension in-tree (python -m morph_amd.build).
 
 Flags that matter for results:
   -ffp-contract=off       no implicit multiply-add fusion: the kernels round
@@ -12,12 +12,15 @@ Flags that matter for results:
 import os
 import subprocess
 import sys
+import sysconfig
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 SOURCES = ["abi.hip", "adamw.hip", "nonfinite.hip", "step.hip", "grads.hip", "convert.hip", "fp8.hip", "gemm.hip", "muon.hip", "muon_small.hip", "hostcopy.hip"]
 OUTPUT = PKG / "lib" / "libmorph_optim.so"
+HOSTPATH = PKG / "lib" / "_hostpath.so"  # Python extension over torch's C++ tensors (hostpath.cpp)
 ARCH = os.environ.get("MORPH_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = [
@@ -31,6 +34,34 @@ FLAGS = [
 def hipcc():
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     return str(Path(rocm) / "bin" / "hipcc")
+
+
+def build_hostpath(output=HOSTPATH):
+    import torch
+    from torch.utils import cpp_extension
+    output = Path(output)
+    output.parent.mkdir(parents=True, exist_ok=True)
+    tmp = output.with_name(output.name + ".tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{p}" for p in cpp_extension.include_paths()],
+           f"-isystem{sysconfig.get_paths()['include']}", "-o", str(tmp),
+           str(PKG / "csrc" / "hostpath.cpp"), f"-L{Path(torch.__file__).parent / 'lib'}",
+           "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        sys.stderr.write(proc.stdout + proc.stderr)
+        raise RuntimeError(f"g++ failed ({proc.returncode}): {' '.join(cmd)}")
+    os.replace(tmp, output)
+    return output
+
+
+def build_all():
+    """The library and the host extension, compiled side by side."""
+    with ThreadPoolExecutor(2) as pool:
+        host = pool.submit(build_hostpath)
+        library = build(quiet=False)
+        return library, host.result()
 
 
 def build(output=OUTPUT, extra_flags=(), quiet=True):
@@ -52,4 +83,4 @@ def build(output=OUTPUT, extra_flags=(), quiet=True):
 
 
 if __name__ == "__main__":
-    print(build(quiet=False))
+    print(*build_all())

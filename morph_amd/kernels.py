@@ -105,8 +105,9 @@ class AdamwBatch:
             d.numel = p.numel()
             d.hp_index = hp_index[i]
             d.clock_index = clock_index[i]
-            keep.append((p, m, v, g, o))
+            keep.append((p, m, v, o))
         self._keep = keep  # the tensors must outlive the descriptors
+        self._grads = list(grads)
         self._table = self._device_table() if n > _lib.ADAMW_LAUNCH_TENSORS else None
         self._grad_dtype = grads[0].dtype if n else None
         self._numels = [p.numel() for p in params]
@@ -172,8 +173,27 @@ class AdamwBatch:
                 raise ValueError(f"grad[{i}] does not match the batch (dtype, size or device)")
         for i, g in enumerate(grads):
             self.array[i].grad = g.data_ptr()
-            p, m, v, _, o = self._keep[i]
-            self._keep[i] = (p, m, v, g, o)
+        self._grads = grads
+
+    def step_plan(self, params, present, clocks, state):
+        """A StepPlan over this batch (hostpath.cpp): params, every parameter in order;
+        present, the indices that the batch steps.  It writes the gradients' addresses into
+        this batch's descriptors and holds the gradients itself."""
+        require_device_tensor(clocks, "clocks")
+        require_device_tensor(state, "state")
+        return _lib.hostpath().StepPlan(
+            list(params), list(present), ctypes.addressof(self.array), self.grad_dtype,
+            self.out_dtype, self._table.data_ptr() if self._table is not None else 0,
+            clocks.data_ptr(), state.data_ptr(),
+            [_lib.entry_address(name) for name in (
+                "morph_nonfinite_or_multi", "morph_nonfinite_or_close", "morph_adamw_multi_dev",
+                "morph_nonfinite_table", "morph_adamw_table_dev")])
+
+    def handed_over(self, stream):
+        """A StepPlan holds the gradients from here on; the table is read on `stream`."""
+        self._grads = None
+        if self._table is not None:
+            self._use_table(stream)
 
     def launch(self, hps, skip_flag=None, stream=None, events=None):
         """Enqueue the step.  hps: sequence of AdamwHP, indexed by hp_index; events:

@@ -21,9 +21,11 @@ multiplies a loss by the device scale without waiting.  With sync=True (or
 on_overflow="raise") every step resolves and reports its outcome like the
 reference does.
 """
+import ctypes
+
 import torch
 
-from . import kernels
+from . import _lib, kernels
 from .control import BiasTables, StepControl
 from .hyper import adamw_constants
 from .precision import DynamicLossScale
@@ -145,9 +147,13 @@ class FusedAdamW:
             loss_scale.attach(self)
         self._dirty = False     # steps enqueued since the host last read the device state
         self._tables = {}
-        self._bound = [0] * len(flat)  # upper bound of each device clock
+        self._bound = 0  # upper bound of every device clock
         self._cache_key = None
         self._cache = None
+        self._plan = None       # hostpath.StepPlan over the cached batch, from its second step on
+        self._plan_key = None   # the cache key it was built for
+        self._consts = None     # (hyperparameters, constants, schedules, table limit) of the groups
+        _lib.hostpath()         # a missing build fails here
         self._slot = 0          # found_inf word of the next step (steps alternate)
         self._pending = None    # (slot, clock_list, stream) of a step whose close is not enqueued
         self.kernel_timer = None  # optional list: (start, end) events around each AdamW launch
@@ -239,10 +245,12 @@ class FusedAdamW:
         return self._tables[key]
 
     def _prepare(self, grads, present):
-        """Descriptor batch, per-group constants and clock list for this set of tensors."""
+        """Descriptor batch, clock list and parameter groups for this set of tensors."""
         flat = self._flat()
         groups = sorted({flat[i][0] for i in present})
         hp_of = {gi: k for k, gi in enumerate(groups)}
+        if self._plan is not None:
+            self._plan.release()
         key = (tuple(present), tuple(grads[i].dtype for i in present),
                tuple(e.data_ptr() for e in self.exports) if self.exports else None)
         ptrs = tuple(grads[i].data_ptr() for i in present)
@@ -254,28 +262,50 @@ class FusedAdamW:
                 [self.exports[i] for i in present] if self.exports else None,
                 hp_index=[hp_of[flat[i][0]] for i in present], clock_index=list(present))
             clock_list = torch.tensor(present, dtype=torch.int32).to(self.device)
-            self._cache = [batch, clock_list, ptrs]
+            self._cache = [batch, clock_list, ptrs, groups]
             self._cache_key = key
-        elif ptrs != self._cache[2]:
+            self._plan = None
+            return batch, clock_list, groups
+        if self._plan is None and self._staging is None:
+            # the same tensors again: their next steps can take the native path
+            self._plan = self._cache[0].step_plan([p for _, p in flat], present, self._ctl.clocks,
+                                                  self._ctl.state)
+            self._plan_key = self._cache_key
+        if ptrs != self._cache[2]:
             # same tensors, new gradient buffers: swap pointers only (no table rebuild,
             # no host-to-device copy that would wait for the queued steps)
             self._cache[0].rebind_grads([grads[i] for i in present])
             self._cache[2] = ptrs
-        batch, clock_list, _ = self._cache
-        hps, scheds = [], []
+        return self._cache[0], self._cache[1], groups
+
+    def _constants(self, groups):
+        """Constant sets and schedules of the listed parameter groups as ctypes arrays, computed
+        again when a hyperparameter has another value or a bias table has to grow."""
+        values = []
+        for gi in groups:
+            g = self.param_groups[gi]
+            beta1, beta2 = g["betas"]
+            values += (gi, g["lr"], beta1, beta2, g["eps"], g["weight_decay"])
+        need = self._bound + 1
+        plain = all(type(v) is float or type(v) is int for v in values)
+        if plain and self._consts is not None and self._consts[0] == values and need <= self._consts[3]:
+            return self._consts[1:3]
+        hps, scheds, limit = [], [], None
         for gi in groups:
             group = self.param_groups[gi]
             beta1, beta2 = group["betas"]
             hps.append(adamw_constants(lr=group["lr"], beta1=beta1, beta2=beta2, eps=group["eps"],
                                        weight_decay=group["weight_decay"], step=1))
             table = self._table(group["betas"])
-            need = max(self._bound[i] for i in present if flat[i][0] == gi) + 1
             table.ensure(need)
             scheds.append(table.sched(group["lr"]))
-        return batch, clock_list, hps, scheds
+            limit = table.length if limit is None else min(limit, table.length)
+        hps = (_lib.AdamwHP * len(hps))(*hps)
+        scheds = (_lib.AdamwSched * len(scheds))(*scheds)
+        self._consts = (values, hps, scheds, limit) if plain else None
+        return hps, scheds
 
     # -- the step ----------------------------------------------------------
-    @torch.no_grad()
     def step(self, grads=None, stream=None, checked=False):
         """Enqueue one optimizer step: the detector (carrying the previous step's
         close), then the fused AdamW pass.  This step's close follows with the next
@@ -289,6 +319,17 @@ class FusedAdamW:
         gradients and masters and returns once the updated masters are back in
         the CPU tensors.
         """
+        # the same parameters and kinds of gradients as last time (all looked at again):
+        # the batch's descriptors are up to date and the launches go out natively
+        if (self._plan is not None and self._plan_key is self._cache_key
+                and self.kernel_timer is None and self.dispatch_timer is None
+                and self._plan.match(self.param_groups, grads, self.exports)):
+            self._cache[2] = None  # the descriptors' addresses are the plan's now
+            return self._enqueue(None, None, stream, checked, planned=True)
+        return self._step(grads, stream, checked)
+
+    @torch.no_grad()
+    def _step(self, grads, stream, checked):
         flat = self._flat()
         if grads is None:
             grads = [p.grad for _, p in flat]
@@ -396,11 +437,10 @@ class FusedAdamW:
         self._chunk_cache = (key, batches)
         return batches
 
-    def _enqueue(self, grads, present, stream, checked, pipeline=False):
+    def _enqueue(self, grads, present, stream, checked, pipeline=False, planned=False):
         """The device step over device gradients (see step()).  pipeline: CPU
         masters, streamed through the update by HostStaging.pipeline (the launch
-        timers do not apply)."""
-        flat = self._flat()
+        timers do not apply).  planned: the plan has matched this step's gradients."""
         if self._ctl.scaler_changed():
             # the caller set the scaler (scale, good_steps, load_state_dict) since the last
             # step: wait for the queued steps, then the caller's values replace what they
@@ -411,15 +451,20 @@ class FusedAdamW:
             finally:
                 self._ctl.restore_host_fields(fields)
             self._ctl.push_scale()
-        batch, clock_list, hps, scheds = self._prepare(grads, present)
+        if planned:
+            batch, clock_list, _, groups = self._cache
+        else:
+            batch, clock_list, groups = self._prepare(grads, present)
+        hps, scheds = self._constants(groups)
         # everything that can fail is done before the first launch is enqueued
         events = self.dispatch_timer.next() if self.dispatch_timer is not None else None
         ctl = self._ctl
         slot = self._slot
-        s = stream or torch.cuda.current_stream(self.device)
-        for table in self._tables.values():
-            table.used_on(s)
-        if s != torch.cuda.current_stream(self.device):
+        current = torch.cuda.current_stream(self.device)
+        s = stream or current
+        if s != current:
+            for table in self._tables.values():
+                table.used_on(s)
             clock_list.record_stream(s)  # allocated on the current stream, read on `s`
         if self._pending is not None and self._pending[2] != s:
             # the previous step ran on another stream: close it there, and order
@@ -429,13 +474,22 @@ class FusedAdamW:
             s.wait_stream(prev)
         if checked:
             self._flush_close()
-        else:
+        if planned:
+            prev = self._pending[1] if self._pending is not None else None
+            batch.handed_over(s)
+            kernels.check(self._plan.launch(
+                s.cuda_stream, slot, checked, prev.data_ptr() if prev is not None else 0,
+                prev.numel() if prev is not None else 0, ctypes.addressof(hps),
+                ctypes.addressof(scheds), len(hps)))
+            self._pending = None
+        elif not checked:
             prev = self._pending[1] if self._pending is not None else None
             batch.detect([grads[i] for i in present], ctl.state, slot, ctl.clocks, prev, s)
             self._pending = None
-        if pipeline:
+        if planned:
+            pass
+        elif pipeline:
             flat = self._flat()
-            groups = sorted({flat[i][0] for i in present})
             chunk_batches = self._chunk_batches(grads, present, {g: k for k, g in enumerate(groups)})
             launches = iter(chunk_batches)
             self._staging.pipeline(
@@ -455,8 +509,7 @@ class FusedAdamW:
         self._pending = (slot, clock_list, s)
         self._slot = slot ^ 1
         self._dirty = True
-        for i in present:
-            self._bound[i] += 1
+        self._bound += 1
         if not self.sync:
             return None
         st = self.resolve()
@@ -505,7 +558,7 @@ class FusedAdamW:
         clocks = self._ctl.clocks.cpu().tolist()
         for i, (_, p) in enumerate(self._flat()):
             self.state[p]["step"] = clocks[i]
-            self._bound[i] = clocks[i]
+        self._bound = max(clocks)
         self.skipped_steps = int(st.skipped)
         self.applied_steps = int(st.applied)
         self._ctl.mirror(st)
@@ -556,6 +609,6 @@ class FusedAdamW:
                 st["exp_avg"].copy_(saved["exp_avg"])
                 st["exp_avg_sq"].copy_(saved["exp_avg_sq"])
             clocks.append(st["step"])
-            self._bound[i] = st["step"]
+        self._bound = max(clocks)
         self._ctl.clocks.copy_(torch.tensor(clocks, dtype=torch.int64))
         self._cache_key = None

@@ -8,6 +8,7 @@ Bit-exact against the oracle everywhere; against torch.optim.AdamW the moments
 are bit-exact and masters agree to max|dw|/max|w| <= 1e-6 (torch's CPU sqrt is
 not correctly rounded; see tests/test_oracle_adamw.py).
 """
+import copy
 import json
 
 import numpy as np
@@ -545,6 +546,59 @@ def test_descriptor_table_equals_kernel_argument_launches(monkeypatch, dtype, ex
     strided = torch.zeros(2 * sizes[0], dtype=dtype, device=DEV)[::2]
     with pytest.raises(ValueError, match="contiguous"):
         a.step([strided] + [torch.zeros(n, dtype=dtype, device=DEV) for n in sizes[1:]])
+
+
+@pytest.mark.parametrize("count", [5, 60])
+def test_native_steps_equal_python_steps(count):
+    """From a batch's second step on the launches go out natively (hostpath.cpp).  A sequence that
+    takes that path and leaves it -- new buffers, missing gradients, another learning rate,
+    checked steps, another stream, overflows, replaced export buffers, a loaded state -- against
+    the same sequence kept on the Python path (an optimizer with a launch timer)."""
+    gen = torch.Generator().manual_seed(7)
+    shapes = [(int(torch.randint(1, 3000, (1,), generator=gen)),) for _ in range(count - 1)] + [(40, 30)]
+    masters = [torch.randn(s, generator=gen) * .02 for s in shapes]
+    steps = [[(torch.randn(s, generator=gen) * 1e-3 * 1024).half() for s in shapes] for _ in range(14)]
+    steps[4][1][0] = float("inf")
+    steps[9][-1][3, 3] = float("nan")
+    side = torch.cuda.Stream()
+    runs, native = [], 0
+    for timed in (False, True):
+        ps = [m.to(DEV) for m in masters]
+        opt = FusedAdamW([dict(params=ps[:2]), dict(params=ps[2:], weight_decay=0.0)], lr=1e-3,
+                         loss_scale=DynamicLossScale(1024.0, growth_interval=4), export_dtype=torch.float16)
+        for k, gs in enumerate(steps):
+            if timed:
+                opt.kernel_timer = []
+            gs = [g.to(DEV) for g in gs]
+            if k in (5, 6):
+                gs[2] = None
+            if k == 7:
+                opt.param_groups[1]["lr"] = 5e-4
+            if k == 8:
+                opt.set_exports([torch.zeros_like(e) for e in opt.exports])
+            if k == 11:
+                opt.load_state_dict(copy.deepcopy(opt.state_dict()))
+            if k == 12:
+                side.wait_stream(torch.cuda.current_stream())
+                opt.step(gs, stream=side)
+                torch.cuda.current_stream().wait_stream(side)
+            else:
+                if k == 10:  # flagged by the gradients' producer
+                    opt.found_inf.fill_(0)
+                opt.step(gs, checked=k == 10)
+            native += not timed and opt._cache[2] is None
+        opt.resolve()
+        runs.append((opt, ps))
+    (a, pa), (b, pb) = runs
+    assert native == 5  # steps 2, 3, 4, 10 and 13
+    assert a.skipped_steps == b.skipped_steps == 2 and a.applied_steps == b.applied_steps
+    assert a.loss_scale.state_dict() == b.loss_scale.state_dict()
+    for p, q, e, f in zip(pa, pb, a.exports, b.exports):
+        assert torch.equal(p, q) and torch.equal(e, f)
+        assert torch.equal(a.state[p]["exp_avg_sq"], b.state[q]["exp_avg_sq"])
+        assert a.state[p]["step"] == b.state[q]["step"]
+    with pytest.raises(ValueError, match="contiguous"):
+        a.step([torch.zeros(2 * g.numel(), dtype=torch.half, device=DEV)[::2] for g in gs])
 
 
 @pytest.mark.parametrize("count,size", [(1, 1 << 24), (200, 1 << 16)], ids=["one", "split"])

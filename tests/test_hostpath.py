@@ -1,0 +1,121 @@
+"""StepPlan.match (hostpath.cpp): which steps the native path takes, on CPU tensors.
+
+match() may say yes only when the Python path would step exactly the batch's tensors with
+these gradients: everything else is its refusal, after which the Python path rebuilds the
+batch or raises.  No launch here: the entry points' addresses are never called.
+"""
+import pytest
+import torch
+
+from morph_amd import _lib
+
+SHAPES = [(4, 6), (5,), (0,), (3, 3)]
+
+
+class Case:
+    """Four parameters in two groups, a batch over all but the second."""
+
+    def __init__(self, dtype=torch.float32, exports=False):
+        self.params = [torch.nn.Parameter(torch.zeros(s)) for s in SHAPES]
+        self.groups = [dict(params=self.params[:2], lr=1.0), dict(params=self.params[2:], lr=2.0)]
+        self.present = [0, 2, 3]
+        self.dtype = dtype
+        self.exports = [torch.zeros(s, dtype=torch.float16) for s in SHAPES] if exports else []
+        self.array = (_lib.AdamwTensor * 3)()
+        for d, i in zip(self.array, self.present):
+            d.numel = self.params[i].numel()
+            d.out = self.exports[i].data_ptr() if exports else None
+        self.plan = _lib.hostpath().StepPlan(self.params, self.present, _lib.ctypes.addressof(self.array),
+                                             _lib.dtype_code(dtype), -1, 0, 0, 0, [0] * 5)
+
+    def grads(self):
+        return [torch.ones(s, dtype=self.dtype) if i in self.present else None
+                for i, s in enumerate(SHAPES)]
+
+    def match(self, grads=None):
+        before = [d.grad for d in self.array]
+        ok = self.plan.match(self.groups, grads, self.exports)
+        if not ok:
+            assert [d.grad for d in self.array] == before  # a refusal writes nothing
+        return ok
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", [list, tuple])
+def test_matching_gradients_are_taken_by_address(dtype, kind):
+    c = Case(dtype, exports=True)
+    for _ in range(2):
+        gs = c.grads()
+        assert c.match(kind(gs))
+        assert [d.grad or 0 for d in c.array] == [gs[i].data_ptr() for i in c.present]
+    address = gs[0].data_ptr()
+    del gs  # the plan holds them until the next match or release()
+    assert torch.ones(4, 6, dtype=dtype).data_ptr() != address
+    c.plan.release()
+
+
+def test_the_parameters_own_gradients():
+    c = Case()
+    for i in c.present:
+        c.params[i].grad = torch.ones_like(c.params[i])
+    assert c.match()
+    assert c.array[0].grad == c.params[0].grad.data_ptr()
+    c.params[1].grad = torch.ones(5)
+    assert not c.match()  # a gradient more
+    c.params[1].grad = None
+    assert c.match()
+    c.params[3].grad = None
+    assert not c.match()  # one less
+
+
+@pytest.mark.parametrize("change", [
+    lambda c, g: g.__setitem__(0, None), lambda c, g: g.__setitem__(1, torch.ones(5)),
+    lambda c, g: g.__setitem__(0, g[0].half()), lambda c, g: g.__setitem__(0, torch.ones(6, 4).t()),
+    lambda c, g: g.__setitem__(0, torch.ones(4, 12)[:, ::2]), lambda c, g: g.__setitem__(3, torch.ones(8)),
+    lambda c, g: g.__setitem__(3, torch.ones(10)), lambda c, g: g.__setitem__(3, g[3].to("meta")),
+    lambda c, g: g.__setitem__(3, g[3].to_sparse()), lambda c, g: g.__setitem__(3, 1.0),
+    lambda c, g: g.__setitem__(3, g[3].expand(1, 3, 3).expand(2, 3, 3)[:, 0]),
+    lambda c, g: g.__setitem__(3, torch.ones(3, 3).as_subclass(type("Sub", (torch.Tensor,), {}))),
+    lambda c, g: g.append(None), lambda c, g: g.pop(),
+    lambda c, g: c.groups.reverse(), lambda c, g: c.groups.pop(),
+    lambda c, g: c.groups[0]["params"].append(torch.nn.Parameter(torch.zeros(2))),
+    lambda c, g: c.groups[1].__setitem__("params", [torch.nn.Parameter(p.data) for p in c.params[2:]]),
+    lambda c, g: c.groups[1].__setitem__("params", tuple(c.params[2:])),
+    lambda c, g: c.exports.__setitem__(3, torch.zeros(3, 3, dtype=torch.float16)),
+    lambda c, g: c.exports.clear(), lambda c, g: c.exports.pop(),
+], ids=range(22))
+def test_anything_else_is_refused(change):
+    c = Case(exports=True)
+    gs = c.grads()
+    assert c.match(gs)
+    change(c, gs)
+    assert not c.match(gs)
+
+
+def test_other_containers_are_refused():
+    c = Case()
+    gs = c.grads()
+    assert not c.match(iter(gs)) and not c.match(dict(enumerate(gs)))
+    assert not c.plan.match(tuple(dict(g, params=iter(g["params"])) for g in c.groups), gs, [])
+    assert c.match(gs)
+
+
+def test_other_views_with_the_same_layout_match():
+    """A contiguous gradient of the right size is taken whatever its shape or offset, as in the
+    Python path."""
+    c = Case()
+    gs = c.grads()
+    gs[0] = torch.ones(24)
+    gs[3] = torch.ones(10)[1:]
+    assert c.match(gs) and c.array[2].grad == gs[3].data_ptr()
+
+
+def test_bad_plans_raise():
+    p = [torch.zeros(3)]
+    make = lambda present, entries=5: _lib.hostpath().StepPlan(  # noqa: E731
+        p, present, _lib.ctypes.addressof((_lib.AdamwTensor * 2)()), 0, -1, 0, 0, 0, [0] * entries)
+    for bad in ([], [1], [0, 0], [-1]):
+        with pytest.raises(ValueError):
+            make(bad)
+    with pytest.raises(ValueError):
+        make([0], 4)
