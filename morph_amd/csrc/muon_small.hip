@@ -34,6 +34,24 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
+// Row and column of the items i0, i0 + step, ... of rows of per_row items each: two
+// divisions in all instead of one per item (about 40 instructions, which took longer than
+// the rest of a pass over the matrix).
+struct Walk {
+  int r, c, dr, dc, per_row;
+  __device__ Walk(int i0, int step, int per_row_) : per_row(per_row_) {
+    r = i0 / per_row;
+    c = i0 - r * per_row;
+    dr = step / per_row;
+    dc = step - dr * per_row;
+  }
+  __device__ void next() {
+    r += dr;
+    c += dc;
+    if (c >= per_row) c -= per_row, ++r;
+  }
+};
+
 // Four consecutive elements of one matrix: torch's lerp roundings, as momentum_one.
 template <bool kMomentum>
 __device__ __forceinline__ float blend(float g, float& m, float mom_w, float nest_w) {
@@ -63,9 +81,10 @@ __global__ __launch_bounds__(kPrep) void small_prepare_kernel(const SmallBatch b
   double ss = 0.0;
   bool bad = false;
   if ((addr & 15) == 0 && (cols & 3) == 0) {
-    const int quads = rows * cols / 4, per_row = cols / 4;
+    const int quads = rows * cols / 4;
+    Walk w(tid, kPrep, cols / 4);
 #pragma unroll 4
-    for (int i = tid; i < quads; i += kPrep) {
+    for (int i = tid; i < quads; i += kPrep, w.next()) {
       const f32x4 gv = reinterpret_cast<const f32x4*>(g)[i];
       f32x4 mv = f32x4{0.f, 0.f, 0.f, 0.f};
       if constexpr (kMomentum) mv = reinterpret_cast<const f32x4*>(mom)[i];
@@ -81,19 +100,18 @@ __global__ __launch_bounds__(kPrep) void small_prepare_kernel(const SmallBatch b
         ss += (double)u * (double)u;
       }
       if constexpr (kMomentum) reinterpret_cast<f32x4*>(mom_out)[i] = mv;
-      const int r = i / per_row, c = (i - r * per_row) * 4;
-      *reinterpret_cast<u32x2*>(x + r * ld + c) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+      *reinterpret_cast<u32x2*>(x + w.r * ld + w.c * 4) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
     }
   } else {
+    Walk w(tid, kPrep, cols);
 #pragma unroll 4
-    for (int i = tid; i < rows * cols; i += kPrep) {
+    for (int i = tid; i < rows * cols; i += kPrep, w.next()) {
       const float gi = g[i];
       bad |= nonfinite_f32_bits(__builtin_bit_cast(uint32_t, gi));
       float m = kMomentum ? mom[i] : 0.f;
       const float u = blend<kMomentum>(gi, m, mom_w, nest_w);
       if constexpr (kMomentum) mom_out[i] = m;
-      const int r = i / cols, c = i - r * cols;
-      x[r * ld + c] = (uint16_t)float_to_bf16_bits(u);
+      x[w.r * ld + w.c] = (uint16_t)float_to_bf16_bits(u);
       ss += (double)u * (double)u;
     }
   }
@@ -134,8 +152,6 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
                                                                 const SmallChain ch) {
   __shared__ __attribute__((aligned(16))) uint16_t lds[kSmallLds / 2];
   constexpr int mp = MB * 32, lda = mp + 8;
-  constexpr int kSym = MB * (MB + 1) / 2;                  // upper triangle of A's tiles
-  constexpr int kSymPer = (kSym + kWaves - 1) / kWaves;    // of them per wave
   constexpr int kCB = column_blocks<MB>();
   const int mat = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -149,22 +165,57 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
   for (int i = tid; i < mp * ldx / 8; i += kChain)
     reinterpret_cast<u32x4*>(X)[i] = u32x4{0u, 0u, 0u, 0u};
   __syncthreads();
+  // A wave covers 16 rows x 4 pieces of a tall matrix at a time: its transposed LDS
+  // accesses then fall on few banks twice, where whole rows of pieces would put 8 lanes on
+  // one bank (470 x 128: 34 K cycles of loading).
+  const int tile_r = lane >> 2, tile_c = lane & 3;
   {
     const int rows = tall ? n : m, cols = tall ? m : n, ld = (cols + 7) & ~7, per_row = ld / 8;
     const uint16_t* x0 = b.x0 + mat * b.stride;
-#pragma unroll 4
-    for (int i = tid; i < rows * per_row; i += kChain) {
-      const int r = i / per_row, c = (i - r * per_row) * 8;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(x0 + r * ld + c);
-      if (!tall && c + 8 <= cols) {
-        *reinterpret_cast<u32x4*>(X + r * ldx + c) = v;
-      } else {
+    constexpr int kBatch = 8;  // loads in flight per lane
+    // elements c .. c + 7 of a row, those past the row zero
+    auto tail = [&](u32x4 v, int c) {
+      const int left = cols - c;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint16_t h = (uint16_t)((e & 1) ? v[e >> 1] >> 16 : v[e >> 1]);
-          if (c + e < cols) {
-            if (tall) X[(c + e) * ldx + r] = h;
-            else X[r * ldx + c + e] = h;
+      for (int k = 0; k < 4; ++k)
+        v[k] &= left >= 2 * k + 2 ? 0xFFFFFFFFu : left == 2 * k + 1 ? 0xFFFFu : 0u;
+      return v;
+    };
+    if (!tall) {
+      const int total = rows * per_row;
+      Walk get(tid, kChain, per_row), put = get;
+      for (int i0 = tid; i0 < total; i0 += kBatch * kChain) {
+        u32x4 v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k, get.next())
+          if (i0 + k * kChain < total)
+            v[k] = *reinterpret_cast<const u32x4*>(x0 + get.r * ld + get.c * 8);
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k, put.next())
+          if (i0 + k * kChain < total)
+            *reinterpret_cast<u32x4*>(X + put.r * ldx + put.c * 8) = tail(v[k], put.c * 8);
+      }
+    } else {
+      const int tiles_c = (per_row + 3) / 4, tiles = (rows + 15) / 16 * tiles_c;
+      Walk get(wave, kWaves, tiles_c), put = get;
+      for (int t0 = wave; t0 < tiles; t0 += kBatch * kWaves) {
+        u32x4 v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k, get.next()) {
+          const int r = get.r * 16 + tile_r, c = get.c * 4 + tile_c;
+          if (t0 + k * kWaves < tiles && r < rows && c < per_row)
+            v[k] = *reinterpret_cast<const u32x4*>(x0 + r * ld + c * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k, put.next()) {
+          const int r = put.r * 16 + tile_r, c = put.c * 4 + tile_c;
+          if (t0 + k * kWaves < tiles && r < rows && c < per_row) {
+            const u32x4 w = tail(v[k], c * 8);  // X row c * 8 + e < round_up(m, 8) <= mp
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const uint32_t word = w[e >> 1];
+              X[(c * 8 + e) * ldx + r] = (uint16_t)((e & 1) ? word >> 16 : word);
+            }
           }
         }
       }
@@ -188,12 +239,6 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
     const u32x2 lo = half(at), hi = half(at + 4 * ldx);
     return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
   };
-  // tile t of the upper triangle, row by row
-  auto tile_of = [](int t, int& i, int& j) {
-    i = 0;
-    while (t >= MB - i) t -= MB - i, ++i;
-    j = i + t;
-  };
   // a symmetric tile and its mirror into A
   auto store_sym = [&](int i, int j, const uint32_t (&w)[8]) {
     uint16_t* at = A + (i * 32 + fr) * lda + j * 32 + 4 * fh;
@@ -207,40 +252,69 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
     }
   };
 
+  // The symmetric products' upper triangle of tiles over the waves: wave w < MB has (w, w)
+  // and the tile of rows w and w + 1 (mod MB), which share their two fragments (at MB = 2
+  // wave 1 has its diagonal alone); at MB = 4 waves 4 and 5 have (0, 2) and (1, 3).  Half
+  // the LDS reads of one tile per wave, and one round.
+  // Tile 0 is (w, w), tile 1 the other, rows ri < rj of blocks.
+  const bool has0 = wave < MB;
+  const bool has1 = MB > 1 && (wave < (MB == 2 ? 1 : MB) || (MB == 4 && wave < 6));
+  const bool wrap = has0 && wave == MB - 1;  // its tile 1 is (0, w)
+  const int ri = wrap ? 0 : has0 ? wave : (has1 ? wave - MB : 0);
+  const int rj = wrap ? MB - 1 : has0 ? wave + 1 : (has1 ? ri + 2 : 0);
+  const int rd = has0 ? wave : 0;
+  auto tile_i = [&](int p) { return p == 0 ? rd : ri; };
+  auto tile_j = [&](int p) { return p == 0 ? rd : rj; };
+  auto has = [&](int p) { return p == 0 ? has0 : has1; };
+  // out[p]: tile p of S S^T over k columns (a multiple of 32); the next two steps'
+  // fragments are read under the current two's MFMAs (the last round reads its own again,
+  // unused).  The Q fragment, the MFMA's first operand, is the tile column's rows.
+  auto product = [&](const uint16_t* S, int ld, int k, f32x16 (&out)[2]) {
+    out[0] = f32x16{};
+    out[1] = f32x16{};
+    if (!has0 && !has1) return;
+    bf16x8 a[2], c[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) a[u] = frag(S, ld, ri * 32, u), c[u] = frag(S, ld, rj * 32, u);
+    for (int kk = 0; kk < k / 16; kk += 2) {
+      const int nk = kk + 2 < k / 16 ? kk + 2 : kk;
+      bf16x8 na[2], nc[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        na[u] = frag(S, ld, ri * 32, nk + u), nc[u] = frag(S, ld, rj * 32, nk + u);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bf16x8 d = wrap ? c[u] : a[u];
+        out[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(d, d, out[0], 0, 0, 0);
+        out[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[u], a[u], out[1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) a[u] = na[u], c[u] = nc[u];
+    }
+  };
+
   for (int it = 0; it < ch.steps; ++it) {
     const float s1 = it == 0 ? b.scale[mat] : 1.0f, s2 = it == 0 ? b.scale[b.count + mat] : 1.0f;
     // A = X X^T (times 1 / den^2 in the first iteration)
+    f32x16 sym[2];
+    product(X, ldx, np, sym);
 #pragma unroll
-    for (int p = 0; p < kSymPer; ++p) {
-      const int t = wave + p * kWaves;
-      if (t < kSym) {
-        int i, j;
-        tile_of(t, i, j);
-        f32x16 acc = f32x16{};
-#pragma unroll 4
-        for (int kk = 0; kk < np / 16; ++kk)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(X, ldx, j * 32, kk),
-                                                        frag(X, ldx, i * 32, kk), acc, 0, 0, 0);
+    for (int p = 0; p < 2; ++p) {
+      if (has(p)) {
         uint32_t w[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) w[k] = pack2(s2 * acc[2 * k], s2 * acc[2 * k + 1]);
-        store_sym(i, j, w);
+        for (int k = 0; k < 8; ++k) w[k] = pack2(s2 * sym[p][2 * k], s2 * sym[p][2 * k + 1]);
+        store_sym(tile_i(p), tile_j(p), w);
       }
     }
     __syncthreads();
     // B' = c A A + b A + a I over A
-    uint32_t bw[kSymPer][8];
+    product(A, lda, mp, sym);
+    uint32_t bw[2][8];
 #pragma unroll
-    for (int p = 0; p < kSymPer; ++p) {
-      const int t = wave + p * kWaves;
-      if (t < kSym) {
-        int i, j;
-        tile_of(t, i, j);
-        f32x16 acc = f32x16{};
-#pragma unroll
-        for (int kk = 0; kk < mp / 16; ++kk)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(A, lda, j * 32, kk),
-                                                        frag(A, lda, i * 32, kk), acc, 0, 0, 0);
+    for (int p = 0; p < 2; ++p) {
+      if (has(p)) {
+        const int i = tile_i(p), j = tile_j(p);
         const uint16_t* at = A + (i * 32 + fr) * lda + j * 32 + 4 * fh;
         float x[16];
 #pragma unroll
@@ -250,7 +324,7 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
           for (int e = 0; e < 4; ++e) {
             const uint32_t w = e & 2 ? d.y : d.x;
             const float dv = bf16_bits_to_float(e & 1 ? w >> 16 : w & 0xFFFFu);
-            x[4 * q + e] = __fmaf_rn(ch.b, dv, ch.c * acc[4 * q + e]);
+            x[4 * q + e] = __fmaf_rn(ch.b, dv, ch.c * sym[p][4 * q + e]);
             if (i == j && fr == 8 * q + 4 * fh + e) x[4 * q + e] = x[4 * q + e] + ch.a;
           }
         }
@@ -260,14 +334,8 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
     }
     __syncthreads();  // every wave has read A
 #pragma unroll
-    for (int p = 0; p < kSymPer; ++p) {
-      const int t = wave + p * kWaves;
-      if (t < kSym) {
-        int i, j;
-        tile_of(t, i, j);
-        store_sym(i, j, bw[p]);
-      }
-    }
+    for (int p = 0; p < 2; ++p)
+      if (has(p)) store_sym(tile_i(p), tile_j(p), bw[p]);
     __syncthreads();
     // X' = B' X (times 1 / den in the first iteration) over X: wave w owns the column
     // blocks w, w + 8, ...
@@ -276,7 +344,7 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
     for (int c = 0; c < kCB; ++c)
 #pragma unroll
       for (int i = 0; i < MB; ++i) acc[c][i] = f32x16{};
-#pragma unroll 2
+#pragma unroll
     for (int kk = 0; kk < mp / 16; ++kk) {
       bf16x8 fa[MB];
 #pragma unroll
@@ -314,39 +382,66 @@ __global__ __launch_bounds__(kChain, 1) void small_chain_kernel(const SmallBatch
   if constexpr (kOut == SmallOut::kStore) {
     uint16_t* x = ch.x + mat * b.stride;
     const int per_row = (n + 7) / 8;
-    for (int i = tid; i < m * per_row; i += kChain) {
-      const int r = i / per_row, c = (i - r * per_row) * 8;
-      *reinterpret_cast<u32x4*>(x + r * ch.ldx + c) = *reinterpret_cast<const u32x4*>(X + r * ldx + c);
-    }
+    Walk w(tid, kChain, per_row);
+    for (int i = tid; i < m * per_row; i += kChain, w.next())
+      *reinterpret_cast<u32x4*>(x + w.r * ch.ldx + w.c * 8) =
+          *reinterpret_cast<const u32x4*>(X + w.r * ldx + w.c * 8);
     return;
   }
-  // the parameter in its stored layout: 4 elements of a row per lane
+  // the parameter in its stored layout: 4 consecutive elements of a row per lane, or one
+  // element per lane when a row or the buffer is not a whole number of 16 bytes
   float* p = b.param[mat];
-  const int rows = tall ? n : m, cols = tall ? m : n, per_row = (cols + 3) / 4;
-  const bool vec = (reinterpret_cast<uintptr_t>(p) & 15) == 0 && (cols & 3) == 0;
+  const int rows = tall ? n : m, cols = tall ? m : n;
   const float scale = ch.scale[mat];
   auto one = [&](float pv, uint32_t u) {
     if constexpr (kOut == SmallOut::kExtract) return bf16_bits_to_float(u);
     else return muon_update_element(pv, u, scale, ch.decay, ch.neg_lr);
   };
-#pragma unroll 4
-  for (int i = tid; i < rows * per_row; i += kChain) {
-    const int r = i / per_row, c = (i - r * per_row) * 4;
-    float* at = p + (int64_t)r * cols + c;
-    uint32_t u[4];
+  auto value = [&](int r, int c) -> uint32_t { return tall ? X[c * ldx + r] : X[r * ldx + c]; };
+  if ((reinterpret_cast<uintptr_t>(p) & 15) == 0 && (cols & 3) == 0) {
+    // 4 consecutive elements per lane: along the rows, or 16 rows x 4 pieces (tile_r, tile_c)
+    // of a tall matrix
+    constexpr int kBatch = 4;
+    const int per_row = cols / 4;
+    const int tiles_c = tall ? (per_row + 3) / 4 : per_row;
+    const int step = tall ? kWaves : kChain, first = tall ? wave : tid;
+    const int total = tall ? (rows + 15) / 16 * tiles_c : rows * per_row;
+    Walk get(first, step, tiles_c), put = get;
+    auto row_of = [&](const Walk& w) { return tall ? w.r * 16 + tile_r : w.r; };
+    auto col_of = [&](const Walk& w) { return tall ? w.c * 4 + tile_c : w.c; };
+    for (int i0 = first; i0 < total; i0 += kBatch * step) {
+      f32x4 v[kBatch];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)  // past the row only inside X's padding
-      u[e] = tall ? X[(c + e) * ldx + r] : X[r * ldx + c + e];
-    if (vec) {
-      f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kOut == SmallOut::kApply) v = *reinterpret_cast<const f32x4*>(at);
+      for (int k = 0; k < kBatch; ++k, get.next()) {
+        const int r = row_of(get), c = col_of(get);
+        v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (kOut == SmallOut::kApply && i0 + k * step < total && r < rows && c < per_row)
+          v[k] = reinterpret_cast<const f32x4*>(p)[r * per_row + c];
+      }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = one(v[e], u[e]);
-      *reinterpret_cast<f32x4*>(at) = v;
-    } else {
+      for (int k = 0; k < kBatch; ++k, put.next()) {
+        const int r = row_of(put), c = col_of(put);
+        if (i0 + k * step < total && r < rows && c < per_row) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < cols) at[e] = one(kOut == SmallOut::kApply ? at[e] : 0.f, u[e]);
+          for (int e = 0; e < 4; ++e) v[k][e] = one(v[k][e], value(r, c * 4 + e));
+          reinterpret_cast<f32x4*>(p)[r * per_row + c] = v[k];
+        }
+      }
+    }
+  } else {
+    constexpr int kBatch = 8;
+    const int total = rows * cols;
+    Walk w(tid, kChain, cols);
+    for (int i0 = tid; i0 < total; i0 += kBatch * kChain) {
+      float v[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        v[k] = 0.f;
+        if (kOut == SmallOut::kApply && i0 + k * kChain < total) v[k] = p[i0 + k * kChain];
+      }
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k, w.next())
+        if (i0 + k * kChain < total) p[i0 + k * kChain] = one(v[k], value(w.r, w.c));
     }
   }
 }
