@@ -67,7 +67,6 @@ static_assert(kGemmMaxApply >= kMaxMats, "a whole batch's update rides on one fu
 //   tile (160 KiB of LDS per CU).
 constexpr int kFlat = 256;
 constexpr int kFlatApply = 64;
-constexpr int kElemsPerBlock = kFlat * 4;
 constexpr int kTR = 64;    // stored rows per momentum transpose tile
 constexpr int kTC = 128;   // stored columns per momentum transpose tile
 constexpr int kATR = 64;   // stored rows per apply transpose tile
@@ -92,6 +91,7 @@ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 struct Layout {
   int64_t rows, cols, m, n, mp, np, count, numel;
+  int64_t quads;   // 4-element pieces of the rows of a matrix stored [m, n]
   int64_t blocks;  // flat blocks per matrix (momentum_kernel)
   int64_t tiles;   // transpose tiles per matrix (momentum_t_kernel)
   int64_t atiles;  // transpose tiles per matrix (apply_t_kernel)
@@ -130,7 +130,8 @@ Layout make_layout(int64_t rows, int64_t cols, int64_t count, int64_t multiple) 
   L.ldn = L.np + kRowPad;
   L.ldm = L.mp + kRowPad;
   L.numel = rows * cols;
-  L.blocks = (L.numel + kElemsPerBlock - 1) / kElemsPerBlock;
+  L.quads = L.m * ((L.n + 3) / 4);
+  L.blocks = (L.quads + kFlat - 1) / kFlat;
   // tiles of a matrix stored with its long side as rows (the ones X transposes)
   L.tiles = ((L.n + kTR - 1) / kTR) * ((L.m + kTC - 1) / kTC);
   L.atiles = ((L.n + kATR - 1) / kATR) * ((L.m + kATC - 1) / kATC);
@@ -206,66 +207,93 @@ __device__ __forceinline__ void flag_nonfinite(uint32_t* found_inf, bool bad) {
     *reinterpret_cast<volatile uint32_t*>(found_inf) = 1u;
 }
 
-// Matrices whose X has the stored layout: a flat pass.  A block covers
-// kElemsPerBlock consecutive elements; a lane moves 4 consecutive elements
-// (one row, pc a multiple of 4) per 128-bit access when the matrix's buffers
-// are 16-byte aligned, else one element per access.  Gradient and momentum
-// are touched once here, so their accesses are non-temporal.
+// Four consecutive elements of a stored row, `left` of them inside the row: one 16-byte
+// access when all are (4-byte aligned: rows of any length and views at any offset; the
+// hardware takes 16-byte accesses at any multiple of 4), else one element at a time.
+typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ f32x4 load_row4(const float* p) {
+  return load_stream<true>(reinterpret_cast<const f32x4_row*>(p));
+}
+
+__device__ __forceinline__ void store_row4(float* p, const f32x4& v) {
+  store_stream<true>(reinterpret_cast<f32x4_row*>(p), (f32x4_row)v);
+}
+
+__device__ __forceinline__ f32x4 load_row4(const float* p, int64_t left) {
+  if (left >= 4) return load_row4(p);
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (left > 0) v.x = p[0];
+  if (left > 1) v.y = p[1];
+  if (left > 2) v.z = p[2];
+  return v;
+}
+
+__device__ __forceinline__ void store_row4(float* p, const f32x4& v, int64_t left) {
+  if (left >= 4) {
+    store_row4(p, v);
+    return;
+  }
+  if (left > 0) p[0] = v.x;
+  if (left > 1) p[1] = v.y;
+  if (left > 2) p[2] = v.z;
+}
+
+// One piece of the momentum pass: the blend, the momentum's new value in m, bf16(u) in h;
+// elements past the row give u = 0 and add nothing.
+template <bool kMomentum>
+__device__ __forceinline__ u32x2 momentum4(const f32x4& g, f32x4& m, int64_t left, float mom_w,
+                                           float nest_w, double& ss, bool& bad) {
+  uint32_t h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float gi = g[e];
+    float mi = m[e], ui;
+    bad |= nonfinite_f32_bits(__builtin_bit_cast(uint32_t, gi));
+    momentum_one<kMomentum>(gi, mi, ui, mom_w, nest_w, mom_w >= 0.5f, nest_w >= 0.5f);
+    if (e >= left) ui = 0.f;
+    m[e] = mi;
+    h[e] = float_to_bf16_bits(ui);
+    ss += (double)ui * (double)ui;
+  }
+  return u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+}
+
+// Row and first column of piece q of rows of `per_row` pieces; 32-bit division where it
+// suffices (a 64-bit one is a hundred instructions).
+__device__ __forceinline__ void piece_of(int64_t q, int64_t per_row, int64_t& r, int64_t& c) {
+  r = q <= (int64_t)0xFFFFFFFF ? (int64_t)((uint32_t)q / (uint32_t)per_row) : q / per_row;
+  c = (q - r * per_row) * 4;
+}
+
+// Matrices whose X has the stored layout ([m, n]): a pass over the rows' 4-element pieces,
+// one per lane: 16-byte accesses of the FP32 streams, 8-byte ones of X, whose rows start
+// on 16 bytes.  Gradient and momentum are touched once here, so their accesses are
+// non-temporal.  Rows that are not a multiple of 4 long (or buffers off 16 bytes) take the
+// same accesses: 8 matrices of 1286 x 4683 148 -> 113 us against one element per lane
+// (apply_flat_kernel: 110 -> 84 us).
 template <bool kMomentum>
 __global__ __launch_bounds__(kFlat) void momentum_kernel(MatPtrs mats, uint16_t* x_all,
-                                                          double* part_all, int64_t rows,
-                                                          int64_t cols, int64_t mp, int64_t ldn,
-                                                          int64_t parts, float mom_w,
-                                                          float nest_w, uint32_t* found_inf) {
+                                                          double* part_all, int64_t m, int64_t n,
+                                                          int64_t mp, int64_t ldn, int64_t parts,
+                                                          float mom_w, float nest_w,
+                                                          uint32_t* found_inf) {
   __shared__ double lds[kFlat / 64];
   const int slot = blockIdx.y, mat = mats.index[slot];
-  const int64_t pc = mats.transposed[slot] ? rows : cols, numel = rows * cols;
-  const float* g = mats.grad[slot];
-  const float* mom = mats.mom[slot];
-  float* mom_out = mats.mom_out[slot];
-  uint16_t* xm = x_all + (int64_t)mat * mp * ldn;
-  const int64_t base = (int64_t)blockIdx.x * kElemsPerBlock;
-  const bool large_m = mom_w >= 0.5f, large_n = nest_w >= 0.5f;
-  const uintptr_t addr = reinterpret_cast<uintptr_t>(g) |
-                         (kMomentum ? reinterpret_cast<uintptr_t>(mom) |
-                                          reinterpret_cast<uintptr_t>(mom_out)
-                                    : 0);
-  const bool vec = (addr & 15) == 0 && (pc & 3) == 0 && base + kElemsPerBlock <= numel;
+  const int64_t per_row = (n + 3) / 4, q = (int64_t)blockIdx.x * kFlat + threadIdx.x;
   double ss = 0.0;
   bool bad = false;
-  if (vec) {
-#pragma unroll
-    for (int k = 0; k < kElemsPerBlock / (4 * kFlat); ++k) {
-      const int64_t i = base + ((int64_t)k * kFlat + threadIdx.x) * 4;
-      const f32x4 gv = load_stream<true>(reinterpret_cast<const f32x4*>(g + i));
-      const u32x4 gb = __builtin_bit_cast(u32x4, gv);
-      bad |= nonfinite_f32_bits(gb.x) | nonfinite_f32_bits(gb.y) | nonfinite_f32_bits(gb.z) |
-             nonfinite_f32_bits(gb.w);
-      f32x4 mv = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kMomentum) mv = load_stream<true>(reinterpret_cast<const f32x4*>(mom + i));
-      uint32_t h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float m = mv[e], ui;
-        momentum_one<kMomentum>(gv[e], m, ui, mom_w, nest_w, large_m, large_n);
-        mv[e] = m;
-        h[e] = float_to_bf16_bits(ui);
-        ss += (double)ui * (double)ui;
-      }
-      if constexpr (kMomentum) store_stream<true>(reinterpret_cast<f32x4*>(mom_out + i), mv);
-      const int64_t r = i / pc, c = i - r * pc;
-      *reinterpret_cast<u32x2*>(xm + r * ldn + c) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-    }
-  } else {
-    for (int64_t i = base + threadIdx.x; i < base + kElemsPerBlock && i < numel; i += kFlat) {
-      float m = kMomentum ? mom[i] : 0.f, ui;
-      bad |= nonfinite_f32_bits(__builtin_bit_cast(uint32_t, g[i]));
-      momentum_one<kMomentum>(g[i], m, ui, mom_w, nest_w, large_m, large_n);
-      if constexpr (kMomentum) mom_out[i] = m;
-      const int64_t r = i / pc, c = i - r * pc;
-      xm[r * ldn + c] = (uint16_t)float_to_bf16_bits(ui);
-      ss += (double)ui * (double)ui;
-    }
+  if (q < m * per_row) {
+    int64_t r, c;
+    piece_of(q, per_row, r, c);
+    const int64_t i = r * n + c, left = n - c;
+    const f32x4 gv = load_row4(mats.grad[slot] + i, left);
+    f32x4 mv = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kMomentum) mv = load_row4(mats.mom[slot] + i, left);
+    // elements past the row are zero padding of X
+    const u32x2 h = momentum4<kMomentum>(gv, mv, left, mom_w, nest_w, ss, bad);
+    if constexpr (kMomentum) store_row4(mats.mom_out[slot] + i, mv, left);
+    *reinterpret_cast<u32x2*>(x_all + (int64_t)mat * mp * ldn + r * ldn + c) = h;
   }
   flag_nonfinite(found_inf, bad);
   const double s = block_sum<kFlat>(ss, lds);
@@ -274,11 +302,10 @@ __global__ __launch_bounds__(kFlat) void momentum_kernel(MatPtrs mats, uint16_t*
 
 // Tile geometry of momentum_t_kernel and apply_t_kernel: tile blockIdx.x
 // of the stored layout [pr, pc] (TR x TC, row-major over tiles), for the
-// matrices whose X is its transpose.  `vec`: a whole tile with dimensions a
-// multiple of 4, moved 4 consecutive elements per lane access.
+// matrices whose X is its transpose.
 struct TileGeo {
   int64_t pr, pc, r0, c0, tiles_c, tile;
-  bool valid, vec;
+  bool valid;
 };
 
 template <int TR, int TC>
@@ -293,10 +320,13 @@ __device__ __forceinline__ TileGeo tile_geo(const MatPtrs& mats, int slot, int64
   t.r0 = (t.tile / t.tiles_c) * TR;
   t.c0 = (t.tile % t.tiles_c) * TC;
   t.valid = t.r0 < t.pr;
-  t.vec = (t.pc & 3) == 0 && (t.pr & 3) == 0 && t.r0 + TR <= t.pr && t.c0 + TC <= t.pc;
   return t;
 }
 
+// Edge tiles and rows that are no multiple of 4 long take the whole tiles' accesses
+// (16 matrices of 4683 x 1286: 535 -> 315 us against one element at a time, the apply pass
+// 646 -> 235 us; 12 of 1000 x 400, partial tiles: 34 -> 20 us and 31 -> 13 us).
+//
 // Matrices whose X is the transpose of the stored layout: the momentum pass
 // per kTR x kTC tile, bf16(u) transposed through LDS so that both the stored
 // reads and the X writes are coalesced.  One partial sum per tile, indexed by
@@ -317,74 +347,51 @@ __global__ __launch_bounds__(kBlock) void momentum_t_kernel(MatPtrs mats, uint16
   const float* mom = mats.mom[slot];
   float* mom_out = mats.mom_out[slot];
   uint16_t* xm = x_all + (int64_t)mat * mp * ldn;
-  const bool large_m = mom_w >= 0.5f, large_n = nest_w >= 0.5f;
-  const uintptr_t addr = reinterpret_cast<uintptr_t>(g) |
-                         (kMomentum ? reinterpret_cast<uintptr_t>(mom) |
-                                          reinterpret_cast<uintptr_t>(mom_out)
-                                    : 0);
-  const bool vec = t.vec && (addr & 15) == 0;
   constexpr int kLPR = kTC / 4, kRPP = kBlock / kLPR;  // stored rows: lanes per row, rows per pass
   constexpr int kPasses = kTR / kRPP;
   const int q = threadIdx.x % kLPR, w = threadIdx.x / kLPR;
   double ss = 0.0;
   bool bad = false;
-  if (vec) {
-    // every load of the tile is issued before the first is used: a lane keeps
-    // 2 x kPasses 128-bit loads in flight, which the few workgroups per CU need
-    // to cover HBM latency
-    f32x4 gv[kPasses], mv[kPasses];
+  // every load of the tile is issued before the first is used: a lane keeps
+  // 2 x kPasses 128-bit loads in flight, which the few workgroups per CU need
+  // to cover HBM latency
+  f32x4 gv[kPasses], mv[kPasses];
+  const int64_t left = t.pc - (t.c0 + 4 * q);
+  auto at = [&](int pass) { return (t.r0 + w + pass * kRPP) * t.pc + t.c0 + 4 * q; };
+  auto in_rows = [&](int pass) { return t.r0 + w + pass * kRPP < t.pr; };
+  // A piece outside the matrix (or at a row's ragged end) loads the matrix's first and drops
+  // it: loads under branches of their own kept the whole tile in copies between them.
+  auto whole = [&](int pass) { return left >= 4 && in_rows(pass); };
+  if (t.pr * t.pc >= 4) {
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass)
-      gv[pass] = load_stream<true>(reinterpret_cast<const f32x4*>(
-          g + (t.r0 + w + pass * kRPP) * t.pc + t.c0 + 4 * q));
+    for (int pass = 0; pass < kPasses; ++pass) gv[pass] = load_row4(g + (whole(pass) ? at(pass) : 0));
+    if constexpr (kMomentum) {
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      mv[pass] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kMomentum)
-        mv[pass] = load_stream<true>(reinterpret_cast<const f32x4*>(
-            mom + (t.r0 + w + pass * kRPP) * t.pc + t.c0 + 4 * q));
+      for (int pass = 0; pass < kPasses; ++pass)
+        mv[pass] = load_row4(mom + (whole(pass) ? at(pass) : 0));
     }
+  }
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      const int rr = w + pass * kRPP;
-      const u32x4 gb = __builtin_bit_cast(u32x4, gv[pass]);
-      bad |= nonfinite_f32_bits(gb.x) | nonfinite_f32_bits(gb.y) | nonfinite_f32_bits(gb.z) |
-             nonfinite_f32_bits(gb.w);
-      uint32_t h[4];
+  for (int pass = 0; pass < kPasses; ++pass) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float m = mv[pass][e], ui;
-        momentum_one<kMomentum>(gv[pass][e], m, ui, mom_w, nest_w, large_m, large_n);
-        mv[pass][e] = m;
-        h[e] = float_to_bf16_bits(ui);
-        ss += (double)ui * (double)ui;
-      }
-      if constexpr (kMomentum)
-        store_stream<true>(reinterpret_cast<f32x4*>(mom_out + (t.r0 + rr) * t.pc + t.c0 + 4 * q),
-                           mv[pass]);
-      *reinterpret_cast<u32x2*>(&tile[rr][4 * q]) =
-          u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    for (int e = 0; e < 4; ++e) {
+      gv[pass][e] = whole(pass) ? gv[pass][e] : 0.f;
+      mv[pass][e] = kMomentum && whole(pass) ? mv[pass][e] : 0.f;
     }
-  } else {
-#pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      const int rr = w + pass * kRPP;
-      const int64_t r = t.r0 + rr, c = t.c0 + 4 * q;
-      uint32_t h[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (r < t.pr && c + e < t.pc) {
-          const int64_t i = r * t.pc + c + e;
-          float m = kMomentum ? mom[i] : 0.f, ui;
-          bad |= nonfinite_f32_bits(__builtin_bit_cast(uint32_t, g[i]));
-          momentum_one<kMomentum>(g[i], m, ui, mom_w, nest_w, large_m, large_n);
-          if constexpr (kMomentum) mom_out[i] = m;
-          h[e] = float_to_bf16_bits(ui);
-          ss += (double)ui * (double)ui;
-        }
-      }
-      *reinterpret_cast<u32x2*>(&tile[rr][4 * q]) =
-          u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    const u32x2 h = momentum4<kMomentum>(gv[pass], mv[pass], 4, mom_w, nest_w, ss, bad);
+    if constexpr (kMomentum)
+      if (whole(pass)) store_row4(mom_out + at(pass), mv[pass]);
+    *reinterpret_cast<u32x2*>(&tile[w + pass * kRPP][4 * q]) = h;
+  }
+  if (left > 0 && left < 4) {  // the piece that ends the rows: one lane in kLPR at most
+#pragma unroll 1
+    for (int pass = 0; pass < kPasses && in_rows(pass); ++pass) {
+      const f32x4 gr = load_row4(g + at(pass), left);
+      f32x4 mr = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kMomentum) mr = load_row4(mom + at(pass), left);
+      const u32x2 h = momentum4<kMomentum>(gr, mr, left, mom_w, nest_w, ss, bad);
+      if constexpr (kMomentum) store_row4(mom_out + at(pass), mr, left);
+      *reinterpret_cast<u32x2*>(&tile[w + pass * kRPP][4 * q]) = h;
     }
   }
   flag_nonfinite(found_inf, bad);
@@ -398,13 +405,9 @@ __global__ __launch_bounds__(kBlock) void momentum_t_kernel(MatPtrs mats, uint16
     uint32_t h[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) h[e] = tile[4 * q2 + e][cc];
-    if (t.vec) {
+    // columns past pr are zero: X's padding
+    if (c < t.pc && r < t.pr)
       *reinterpret_cast<u32x2*>(xm + c * ldn + r) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c < t.pc && r + e < t.pr) xm[c * ldn + r + e] = (uint16_t)h[e];
-    }
   }
   const double s = block_sum(ss, lds);
   if (threadIdx.x == 0) part_all[(int64_t)mat * parts + t.tile] = s;
@@ -421,7 +424,16 @@ __global__ __launch_bounds__(kBlock) void norm_kernel(MatPtrs mats, const double
   const int mat = blockIdx.x;
   const int64_t n = x_is_stored(mats, mat, rows, cols) ? blocks : tiles;
   double s = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += kBlock) s += part_all[(int64_t)mat * parts + i];
+  const double* part = part_all + (int64_t)mat * parts;
+  int64_t i = threadIdx.x;
+  for (; i + 7 * kBlock < n; i += 8 * kBlock) {  // 8 loads in flight, added in index order
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = part[i + k * kBlock];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
+  for (; i < n; i += kBlock) s += part[i];
   const double t = block_sum(s, lds);
   if (threadIdx.x == 0) {
     const float den = (float)sqrt(t) + 1e-7f;
@@ -436,21 +448,17 @@ __global__ __launch_bounds__(kBlock) void norm_kernel(MatPtrs mats, const double
 // whole padded output from its inputs, so X0's padding is the only one a call
 // inherits; the chain writes X0 in its second iteration, and a non-finite
 // input leaves NaN there (0 * NaN), so every prepare restores the zeros.
+// One wave per row, 8 elements per lane and access.
 __global__ __launch_bounds__(kBlock) void pad_zero_kernel(uint16_t* x_all, int64_t m, int64_t n,
                                                           int64_t mp, int64_t np, int64_t ldn) {
-  uint16_t* xm = x_all + (int64_t)blockIdx.y * mp * ldn;
-  const int64_t tail = np - n, per_row = tail > 0 ? tail : 0;
-  const int64_t total = m * per_row + (mp - m) * np;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * kBlock) {
-    if (i < m * per_row) {
-      const int64_t r = i / per_row;
-      xm[r * ldn + n + (i - r * per_row)] = 0;
-    } else {
-      const int64_t j = i - m * per_row, r = m + j / np;
-      xm[r * ldn + (j - (r - m) * np)] = 0;
-    }
-  }
+  const int64_t r = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (r >= mp) return;
+  uint16_t* row = x_all + (int64_t)blockIdx.y * mp * ldn + r * ldn;
+  const int lane = threadIdx.x & 63;
+  const int64_t from = r < m ? n : 0, whole = (from + 7) / 8 * 8;  // np is a multiple of 64
+  if (from + lane < whole) row[from + lane] = 0;
+  for (int64_t c = whole + 8 * lane; c < np; c += 8 * 64)
+    *reinterpret_cast<u32x4*>(row + c) = u32x4{0u, 0u, 0u, 0u};
 }
 
 // Without Newton-Schulz iterations X itself is the result: X = bf16(X0 / den)
@@ -478,40 +486,30 @@ __device__ __forceinline__ float apply_one(float p, uint32_t u16, float scale, f
   }
 }
 
-// Matrices whose X has the stored layout: a flat pass, kFlatApply * 4 consecutive
-// elements of p per block (rows of X read at their padded stride).
+// Matrices whose X has the stored layout: a pass over the rows' 4-element pieces, as
+// momentum_kernel.
 template <bool kExtract>
 __global__ __launch_bounds__(kFlatApply) void apply_flat_kernel(MatPtrs mats,
-                                                                const uint16_t* x_all,
-                                                                int64_t rows, int64_t cols,
-                                                                int64_t mp, int64_t ldn,
+                                                                const uint16_t* x_all, int64_t m,
+                                                                int64_t n, int64_t mp, int64_t ldn,
                                                                 float scale_n, float scale_t,
                                                                 float decay, float neg_lr) {
   const int slot = blockIdx.y, mat = mats.index[slot];
-  const int64_t pc = mats.transposed[slot] ? rows : cols, numel = rows * cols;
-  float* p = mats.param[slot];
+  const int64_t per_row = (n + 3) / 4, q = (int64_t)blockIdx.x * kFlatApply + threadIdx.x;
+  if (q >= m * per_row) return;
+  int64_t r, c;
+  piece_of(q, per_row, r, c);
   const float scale = mats.transposed[slot] ? scale_t : scale_n;
-  const uint16_t* xm = x_all + (int64_t)mat * mp * ldn;
-  const int64_t base = (int64_t)blockIdx.x * kFlatApply * 4;
-  const bool vec = (reinterpret_cast<uintptr_t>(p) & 15) == 0 && (pc & 3) == 0 &&
-                   base + kFlatApply * 4 <= numel;
-  if (vec) {
-    const int64_t i = base + (int64_t)threadIdx.x * 4;
-    const int64_t r = i / pc, c = i - r * pc;
-    const u32x2 v = *reinterpret_cast<const u32x2*>(xm + r * ldn + c);
-    const uint32_t h[4] = {v.x & 0xFFFFu, v.x >> 16, v.y & 0xFFFFu, v.y >> 16};
-    f32x4 pv = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (!kExtract) pv = load_stream<true>(reinterpret_cast<const f32x4*>(p + i));
+  float* p = mats.param[slot] + r * n + c;
+  const u32x2 x = *reinterpret_cast<const u32x2*>(x_all + (int64_t)mat * mp * ldn + r * ldn + c);
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (!kExtract) v = load_row4(p, n - c);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) pv[e] = apply_one<kExtract>(pv[e], h[e], scale, decay, neg_lr);
-    store_stream<true>(reinterpret_cast<f32x4*>(p + i), pv);
-  } else {
-    for (int64_t i = base + threadIdx.x; i < base + kFlatApply * 4 && i < numel;
-         i += kFlatApply) {
-      const int64_t r = i / pc, c = i - r * pc;
-      p[i] = apply_one<kExtract>(kExtract ? 0.f : p[i], xm[r * ldn + c], scale, decay, neg_lr);
-    }
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t w = e & 2 ? x.y : x.x;
+    v[e] = apply_one<kExtract>(v[e], e & 1 ? w >> 16 : w & 0xFFFFu, scale, decay, neg_lr);
   }
+  store_row4(p, v, n - c);
 }
 
 // Matrices whose X is the transpose of the stored layout: per kATR x kATC tile of p,
@@ -529,62 +527,51 @@ __global__ __launch_bounds__(kBlock) void apply_t_kernel(MatPtrs mats, const uin
   float* p = mats.param[slot];
   const float scale = mats.transposed[slot] ? scale_t : scale_n;
   const uint16_t* xm = x_all + (int64_t)mat * mp * ldn;
-  const bool vec = t.vec && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
   constexpr int kLPR = kATC / 4, kRPP = kBlock / kLPR;  // stored rows: lanes per row, rows per pass
+  constexpr int kPasses = kATR / kRPP;
   const int q = threadIdx.x % kLPR, w = threadIdx.x / kLPR;
+  const int64_t left = t.pc - (t.c0 + 4 * q);
+  auto at = [&](int pass) { return p + (t.r0 + w + pass * kRPP) * t.pc + t.c0 + 4 * q; };
+  auto in_rows = [&](int pass) { return t.r0 + w + pass * kRPP < t.pr; };
   // the p rows go out first: they do not wait for the X tile
-  f32x4 pv[kATR / kRPP];
-  if (vec && !kExtract) {
+  // (outside the matrix: its first piece, dropped, as in momentum_t_kernel)
+  auto whole = [&](int pass) { return left >= 4 && in_rows(pass); };
+  f32x4 pv[kPasses];
+  if (!kExtract && t.pr * t.pc >= 4) {
 #pragma unroll
-    for (int pass = 0; pass < kATR / kRPP; ++pass)
-      pv[pass] = load_stream<true>(
-          reinterpret_cast<const f32x4*>(p + (t.r0 + w + pass * kRPP) * t.pc + t.c0 + 4 * q));
+    for (int pass = 0; pass < kPasses; ++pass) pv[pass] = load_row4(whole(pass) ? at(pass) : p);
   }
-  // tile[c - c0][r - r0] = X[c][r]: X rows c0 .. c0 + kATC - 1, columns r0 .. r0 + kATR - 1
+  // tile[c - c0][r - r0] = X[c][r]: X rows c0 .. c0 + kATC - 1, columns r0 .. r0 + kATR - 1,
+  // all loads in flight together, behind the p loads (past pr: X's padding)
   constexpr int kXL = kATR / 4, kXRP = kBlock / kXL, kXPasses = kATC / kXRP;
   const int q2 = threadIdx.x % kXL, w2 = threadIdx.x / kXL;
-  if (t.vec) {
-    // all X loads in flight together, behind the p loads
-    u32x2 xv[kXPasses];
+  u32x2 xv[kXPasses];
 #pragma unroll
-    for (int pass = 0; pass < kXPasses; ++pass)
-      xv[pass] = *reinterpret_cast<const u32x2*>(xm + (t.c0 + w2 + pass * kXRP) * ldn + t.r0 +
-                                                 4 * q2);
-#pragma unroll
-    for (int pass = 0; pass < kXPasses; ++pass)
-      *reinterpret_cast<u32x2*>(&tile[w2 + pass * kXRP][4 * q2]) = xv[pass];
-  } else {
-#pragma unroll
-    for (int pass = 0; pass < kXPasses; ++pass) {
-      const int cc = w2 + pass * kXRP;
-      const int64_t c = t.c0 + cc, r = t.r0 + 4 * q2;
-      uint32_t h[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c < t.pc && r + e < t.pr) h[e] = xm[c * ldn + r + e];
-      *reinterpret_cast<u32x2*>(&tile[cc][4 * q2]) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-    }
+  for (int pass = 0; pass < kXPasses; ++pass) {
+    const int64_t c = t.c0 + w2 + pass * kXRP, r = t.r0 + 4 * q2;
+    xv[pass] = *reinterpret_cast<const u32x2*>(xm + (c < t.pc && r < t.pr ? c * ldn + r : 0));
   }
+#pragma unroll
+  for (int pass = 0; pass < kXPasses; ++pass)
+    *reinterpret_cast<u32x2*>(&tile[w2 + pass * kXRP][4 * q2]) = xv[pass];
   __syncthreads();
+  auto update = [&](f32x4 v, int pass) {
 #pragma unroll
-  for (int pass = 0; pass < kATR / kRPP; ++pass) {
-    const int rr = w + pass * kRPP;
-    const int64_t r = t.r0 + rr, c = t.c0 + 4 * q;
-    uint32_t h[4];
+    for (int e = 0; e < 4; ++e)
+      v[e] = apply_one<kExtract>(kExtract ? 0.f : v[e], tile[4 * q + e][w + pass * kRPP], scale,
+                                 decay, neg_lr);
+    return v;
+  };
 #pragma unroll
-    for (int e = 0; e < 4; ++e) h[e] = tile[4 * q + e][rr];
-    float* pr_ = p + r * t.pc + c;
-    if (vec) {
+  for (int pass = 0; pass < kPasses; ++pass) {
+    if (whole(pass)) store_row4(at(pass), update(pv[pass], pass));
+  }
+  if (left > 0 && left < 4) {  // the piece that ends the rows: one lane in kLPR at most
+#pragma unroll 1
+    for (int pass = 0; pass < kPasses && in_rows(pass); ++pass) {
       f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (!kExtract) v = pv[pass];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = apply_one<kExtract>(v[e], h[e], scale, decay, neg_lr);
-      store_stream<true>(reinterpret_cast<f32x4*>(pr_), v);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (r < t.pr && c + e < t.pc)
-          pr_[e] = apply_one<kExtract>(kExtract ? 0.f : pr_[e], h[e], scale, decay, neg_lr);
+      if (!kExtract) v = load_row4(at(pass), left);
+      store_row4(at(pass), update(v, pass), left);
     }
   }
 }
@@ -632,7 +619,7 @@ int setup(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
   if (reinterpret_cast<uintptr_t>(workspace) % 256) return MORPH_EINVAL;
   // grid x of the tile passes and of apply_flat_kernel (the most blocks of the flat passes)
   if (L.tiles > INT32_MAX || L.atiles > INT32_MAX ||
-      (L.numel + kFlatApply * 4 - 1) / (kFlatApply * 4) > INT32_MAX)
+      (L.quads + kFlatApply - 1) / kFlatApply > INT32_MAX)
     return MORPH_ERANGE;
   char* ws = static_cast<char*>(workspace);
   out->L = L;
@@ -741,8 +728,7 @@ int prepare(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols
   const MatPtrs tiled = pointers(mats, count, rows, cols, Orient::kTransposed, &n_tiled);
   const float mw = hp->momentum_weight, nw = hp->nesterov_weight;
   if (L.mp != L.m || L.np != L.n) {
-    const int64_t pad = L.m * (L.np - L.n) + (L.mp - L.m) * L.np;
-    const int64_t bx = std::min<int64_t>((pad + kBlock - 1) / kBlock, 1024);
+    const int64_t bx = (L.mp + kBlock / 64 - 1) / (kBlock / 64);
     hipLaunchKernelGGL(pad_zero_kernel, dim3((unsigned)bx, count), dim3(kBlock), 0, s, W.X[0],
                        L.m, L.n, L.mp, L.np, L.ldn);
     if ((rc = launch_status())) return rc;
@@ -751,10 +737,10 @@ int prepare(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols
     const dim3 ew((unsigned)L.blocks, n_flat);
     if (orth_only)
       hipLaunchKernelGGL(momentum_kernel<false>, ew, dim3(kFlat), 0, s, flat, W.X[0], W.part,
-                         rows, cols, L.mp, L.ldn, L.parts, mw, nw, found_inf);
+                         L.m, L.n, L.mp, L.ldn, L.parts, mw, nw, found_inf);
     else
       hipLaunchKernelGGL(momentum_kernel<true>, ew, dim3(kFlat), 0, s, flat, W.X[0], W.part,
-                         rows, cols, L.mp, L.ldn, L.parts, mw, nw, found_inf);
+                         L.m, L.n, L.mp, L.ldn, L.parts, mw, nw, found_inf);
     if ((rc = launch_status())) return rc;
   }
   if (n_tiled) {
@@ -866,13 +852,13 @@ int finish(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
                                  first + n);
   const float sn = hp->update_scale, st = hp->update_scale_transposed;
   if (n_flat) {
-    const dim3 ew((unsigned)((L.numel + kFlatApply * 4 - 1) / (kFlatApply * 4)), n_flat);
+    const dim3 ew((unsigned)((L.quads + kFlatApply - 1) / kFlatApply), n_flat);
     if (orth_only)
-      hipLaunchKernelGGL(apply_flat_kernel<true>, ew, dim3(kFlatApply), 0, s, flat, x, rows,
-                         cols, L.mp, L.ldn, sn, st, hp->decay, hp->neg_lr);
+      hipLaunchKernelGGL(apply_flat_kernel<true>, ew, dim3(kFlatApply), 0, s, flat, x, L.m,
+                         L.n, L.mp, L.ldn, sn, st, hp->decay, hp->neg_lr);
     else
-      hipLaunchKernelGGL(apply_flat_kernel<false>, ew, dim3(kFlatApply), 0, s, flat, x, rows,
-                         cols, L.mp, L.ldn, sn, st, hp->decay, hp->neg_lr);
+      hipLaunchKernelGGL(apply_flat_kernel<false>, ew, dim3(kFlatApply), 0, s, flat, x, L.m,
+                         L.n, L.mp, L.ldn, sn, st, hp->decay, hp->neg_lr);
     if ((rc = launch_status())) return rc;
   }
   if (n_tiled) {

@@ -386,6 +386,33 @@ def test_muon_step_elementwise_bitexact(shape, offset):
     assert_same_bits(p.cpu().numpy(), op, "param")
 
 
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("shape", [(129, 259), (259, 129), (131, 262), (262, 131), (200, 515),
+                                   (515, 200), (130, 1), (1, 2600), (2600, 3), (321, 321)])
+def test_ragged_elementwise_passes_bitexact(shape, offset):
+    """The general passes (operands too large for the small path, or a single long row) at widths
+    of every remainder of 4, partial tiles in both directions, views at 4, 8 and 12 bytes: 16-byte
+    accesses at any multiple of 4 and the ragged ends of rows.  Nothing outside the views is
+    written, and a non-finite value in the last element is seen."""
+    test_muon_step_elementwise_bitexact(shape, offset)
+    gen = torch.Generator().manual_seed(3)
+    guard = 64
+    n = shape[0] * shape[1]
+    buf = [torch.full((n + offset + 2 * guard,), 7.0, device=DEV) for _ in range(2)]
+    p, m = (b[guard + offset:guard + offset + n].view(shape) for b in buf)
+    p.zero_()
+    m.zero_()
+    g = on_device(torch.randn(shape, generator=gen) * 1e-3, offset)
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    muon.muon_step([p], [g], [m], .02, .01, found_inf=flag)
+    assert flag.item() == 0
+    for b in buf:
+        assert (b[:guard + offset] == 7).all() and (b[guard + offset + n:] == 7).all()
+    g.view(-1)[-1] = float("inf")
+    muon.muon_step([p], [g], [m], .02, .01, found_inf=flag)
+    assert flag.item() == 1
+
+
 def emulated_muon_step(p, g, m, lr, wd):
     """optimizer.py:55-61 with the oracle's elementwise steps (bit-exact with torch) and
     the bf16 Newton-Schulz emulation: the tolerance reference of the GPU step."""
