@@ -995,7 +995,7 @@ double launch_us(int ts, int64_t tiles, int64_t kt, Epilogue e) {
                                     : 0.5 * n - 0.3;
     return (double)kt * stage + n * (d ? 2.3 : up ? 6.0 : 1.3) + 2.0;
   }
-  return (double)kt * std::max(0.22, 0.24 * q) + 3.0;
+  return (double)kt * std::max(0.22, 0.24 * q) + (up ? 1.2 * q : 0.0) + 3.0;
 }
 
 struct Choice {
@@ -1009,7 +1009,7 @@ struct Choice {
 //   A = X X^T, one 768 x 2048: 39 / 16 / 10; twelve: 41 / 24 / 29; thirty-six: 55 / 54 / 70;
 //   one 3072 x 6144: 102 / 75 / 120; three: 146 / 179 / 352;
 //   X' = B' X, one 3072 x 6144: 128 / 114 / 168; three: 288 / 314 / 505;
-//   its update, thirty-six 768 x 2048: 201 / 182 (256 / 128).
+//   its update, thirty-six 768 x 2048: 201 / 182 / 211.
 Choice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool symmetric, Epilogue e) {
   Choice best{0, 0.0};
   for (int ts = 256; ts >= 64; ts /= 2) {
