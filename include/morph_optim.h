@@ -374,7 +374,7 @@ int morph_fp8_unpack(const uint8_t* bytes, const float* scales, int64_t n, void*
 
 /* ---- Hybrid Muon: Newton-Schulz orthogonalisation on bf16 MFMA ---------- */
 
-/* Tile of morph_gemm_nt_bf16: M and N must be multiples of 256, K of 64. */
+/* morph_gemm_nt_bf16 takes M and N in multiples of 256 and K of 64 (whichever tile it runs). */
 #define MORPH_GEMM_TILE_M 256
 #define MORPH_GEMM_TILE_N 256
 #define MORPH_GEMM_TILE_K 64
@@ -393,11 +393,11 @@ int morph_fp8_unpack(const uint8_t* bytes, const float* scales, int64_t n, void*
  * iteration of optimizer.py:19-21 are all of this form (see gemm.hip).
  * flags: MORPH_GEMM_SYMMETRIC (requires M == N, Ct == NULL, and D symmetric
  * if given): C is known to be symmetric, so only the upper triangle of tiles
- * is computed and each off-diagonal tile is mirrored.  MORPH_GEMM_Q_KN: Q is
+ * (of 256, 128 or 64, by the batch) is computed and each off-diagonal tile is mirrored.  MORPH_GEMM_Q_KN: Q is
  * stored [K, N] (ldq >= N) and the product is P . Q (not with SYMMETRIC).
  * C must not overlap P or Q.  Pointers 16-byte aligned, leading dimensions
  * and strides multiples of 8, at most 2^23; MORPH_ERANGE when a dimension is
- * not a tile multiple.
+ * not such a multiple.
  */
 int morph_gemm_nt_bf16(const uint16_t* P, const uint16_t* Q, const uint16_t* D, uint16_t* C,
                        uint16_t* Ct, int64_t M, int64_t N, int64_t K, int64_t batch,
@@ -442,7 +442,8 @@ typedef struct morph_muon_hp {
   float update_scale_transposed;
 } morph_muon_hp;
 
-/* Workspace bytes morph_muon_step needs for `count` matrices of [rows, cols] (either orientation). */
+/* Workspace bytes morph_muon_step needs for `count` matrices of [rows, cols] (either
+ * orientation): room for operands padded to 256, the most any call pads them. */
 size_t morph_muon_workspace_bytes(int64_t rows, int64_t cols, int count);
 
 /*
@@ -511,12 +512,15 @@ int morph_muon_finish_range(const morph_muon_matrix* mats, int count, int64_t ro
  * morph_muon_newton_schulz followed by morph_muon_finish (the master update,
  * not orthogonalize_only), after morph_muon_prepare, with the same bits.  When
  * the batch's operand has no padding (min(rows, cols) and max(rows, cols)
- * multiples of 256) and every param is 16-byte aligned, the last product
- * X' = B' X updates the parameters in its epilogue instead of storing X' (the
- * update runs while other tiles still compute, and the finish pass's reads of
- * X and p become the epilogue's reads of p); the last iteration's X is then not
- * written to the workspace.  Otherwise the two phases run as they are.
- * morph_muon_step uses it.  Replaces optimizer.py:19-22 and 60-61 for a batch.
+ * multiples of the tile edge the library pads this batch to: 64, 128 or 256) and
+ * every param is 16-byte aligned, the last product X' = B' X updates the
+ * parameters in its epilogue instead of storing X' (the update runs while other
+ * tiles still compute, and the finish pass's reads of X and p become the
+ * epilogue's reads of p).  Matrices that run their whole chain in one workgroup
+ * (min(rows, cols) <= 128, fitting a CU's LDS) are updated by that launch, whatever
+ * the padding and alignment.  In both cases the last iteration's X is not written
+ * to the workspace.  Otherwise the two phases run as they are.  morph_muon_step
+ * uses it.  Replaces optimizer.py:19-22 and 60-61 for a batch.
  */
 int morph_muon_newton_schulz_finish(const morph_muon_matrix* mats, int count, int64_t rows,
                                     int64_t cols, const morph_muon_hp* hp, void* workspace,
