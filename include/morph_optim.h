@@ -526,6 +526,21 @@ int morph_muon_newton_schulz_finish(const morph_muon_matrix* mats, int count, in
                                     int64_t cols, const morph_muon_hp* hp, void* workspace,
                                     size_t workspace_bytes, void* stream);
 
+/*
+ * The same in two calls, for a caller whose step may still be dropped after prepare
+ * (a flag it reads back): _ahead enqueues the chain's first products, as many as cover
+ * about 100 us, so that the device works while the flag travels; they write the
+ * workspace only.  _finish_rest, with the same count, rows, cols, hp and workspace,
+ * enqueues what is left of the chain and the update.  Both together give the bits of
+ * morph_muon_newton_schulz_finish; without _finish_rest no parameter has changed and
+ * the workspace is free for another prepare.
+ */
+int morph_muon_newton_schulz_ahead(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+int morph_muon_newton_schulz_finish_rest(const morph_muon_matrix* mats, int count, int64_t rows,
+                                         int64_t cols, const morph_muon_hp* hp, void* workspace,
+                                         size_t workspace_bytes, void* stream);
+
 /* ---- Host staging copy ---------------------------------------------------
  * dst[0, bytes) <- src[0, bytes) on the host, split over up to `threads`
  * threads (1..64) of a pool the library keeps; the calling thread copies

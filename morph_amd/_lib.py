@@ -34,7 +34,8 @@ EXPORTS = (
     "morph_gemm_nt_bf16",
     "morph_muon_workspace_bytes", "morph_muon_step", "morph_muon_orthogonalize",
     "morph_muon_prepare", "morph_muon_newton_schulz", "morph_muon_finish",
-    "morph_muon_finish_range", "morph_muon_newton_schulz_finish", "morph_host_copy",
+    "morph_muon_finish_range", "morph_muon_newton_schulz_finish",
+    "morph_muon_newton_schulz_ahead", "morph_muon_newton_schulz_finish_rest", "morph_host_copy",
 )
 GEMM_TILE_M, GEMM_TILE_N, GEMM_TILE_K = 256, 256, 64
 GEMM_SYMMETRIC = 1
@@ -172,6 +173,11 @@ def _load():
         "morph_muon_newton_schulz_finish": ([ctypes.POINTER(MuonMatrix), i32, i64, i64,
                                              ctypes.POINTER(MuonHP), vp, ctypes.c_size_t, vp],
                                             i32),
+        "morph_muon_newton_schulz_ahead": ([i32, i64, i64, ctypes.POINTER(MuonHP), vp,
+                                            ctypes.c_size_t, vp], i32),
+        "morph_muon_newton_schulz_finish_rest": ([ctypes.POINTER(MuonMatrix), i32, i64, i64,
+                                                  ctypes.POINTER(MuonHP), vp, ctypes.c_size_t,
+                                                  vp], i32),
         "morph_host_copy": ([vp, vp, ctypes.c_size_t, i32], i32),
     }
     for name, (args, res) in sig.items():

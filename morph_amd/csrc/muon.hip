@@ -775,15 +775,41 @@ bool can_fuse_update(const morph_muon_matrix* mats, int count, const Layout& L) 
   return true;
 }
 
+// How many of a chain's products (three per iteration) may run before the caller knows
+// that the step stands: enough to cover its round trip to the host, about 60 us, by the
+// GEMM's cost rule, which a step that is dropped then wastes; never the last product, which
+// may carry the parameter update.  The one-launch chain of small matrices has none.
+// Both halves of a chain count them anew, so they depend on shape, count and steps only.
+int64_t products_ahead(const Layout& L, int count, const morph_muon_hp* hp) {
+  constexpr double kCoverUs = 100.0;
+  if (hp->ns_steps < 1 || takes_small(L, hp)) return 0;
+  const double us[3] = {gemm_us(L.mp, L.mp, L.np, count, true, false),
+                        gemm_us(L.mp, L.mp, L.mp, count, true, true),
+                        gemm_us(L.mp, L.np, L.mp, count, false, false)};
+  const int64_t most = 3 * (int64_t)hp->ns_steps - 1;
+  int64_t n = 0;
+  for (double t = 0.0; n < most && t < kCoverUs; ++n) t += us[n % 3];
+  return n;
+}
+
+// Which products of the chain a call runs.
+enum class Part { kAll, kAhead, kRest };
+
 // fuse: the batch's matrices, whose parameter update the last product (or the small
 // chain) carries in place of writing X (can_fuse_update must hold); nullptr: X is written.
 int newton_schulz(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp,
                   void* workspace, size_t workspace_bytes, void* stream,
-                  const morph_muon_matrix* fuse = nullptr) {
+                  const morph_muon_matrix* fuse = nullptr, Part part = Part::kAll) {
   Bufs W;
   int rc = setup(nullptr, count, rows, cols, hp, workspace, workspace_bytes, false, false, &W);
   if (rc || count == 0) return rc;
   const Layout& L = W.L;
+  const int64_t ahead = part == Part::kAll ? 0 : products_ahead(L, count, hp);
+  // product p of iteration it is number 3 it + p; this call runs first .. last - 1
+  const int64_t first = part == Part::kRest ? ahead : 0;
+  const int64_t last = part == Part::kAhead ? ahead : 3 * (int64_t)hp->ns_steps;
+  auto runs = [&](int64_t it, int p) { return 3 * it + p >= first && 3 * it + p < last; };
+  if (first >= last) return MORPH_OK;
   if (takes_small(L, hp))
     return run_small_chain(W, fuse, count, hp,
                            fuse != nullptr ? SmallOut::kApply : SmallOut::kStore,
@@ -798,15 +824,21 @@ int newton_schulz(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp
     const float* inv_den = it == 0 ? W.scale : nullptr;
     const float* inv_den2 = it == 0 ? W.scale + count : nullptr;
     // A = X X^T (symmetric: upper triangle of tiles, mirrored)
-    rc = gemm_nt_bf16_scaled(X, X, nullptr, W.A, nullptr, L.mp, L.mp, L.np, count, n, n, 0, m, 0,
-                             sx, sx, 0, ss, 0, 1.0f, 0.0f, inv_den2, 0.0f, MORPH_GEMM_SYMMETRIC,
-                             stream);
+    if (runs(it, 0))
+      rc = gemm_nt_bf16_scaled(X, X, nullptr, W.A, nullptr, L.mp, L.mp, L.np, count, n, n, 0, m, 0,
+                               sx, sx, 0, ss, 0, 1.0f, 0.0f, inv_den2, 0.0f, MORPH_GEMM_SYMMETRIC,
+                               stream);
     if (rc) return rc;
     // B' = c (A A^T) + b A + a I (symmetric; a added on the diagonal before rounding)
-    rc = gemm_nt_bf16_scaled(W.A, W.A, W.A, W.B, nullptr, L.mp, L.mp, L.mp, count, m, m, m, m, 0,
-                             ss, ss, ss, ss, 0, hp->c, hp->b, nullptr, hp->a, MORPH_GEMM_SYMMETRIC,
-                             stream);
+    if (runs(it, 1))
+      rc = gemm_nt_bf16_scaled(W.A, W.A, W.A, W.B, nullptr, L.mp, L.mp, L.mp, count, m, m, m, m, 0,
+                               ss, ss, ss, ss, 0, hp->c, hp->b, nullptr, hp->a,
+                               MORPH_GEMM_SYMMETRIC, stream);
     if (rc) return rc;
+    if (!runs(it, 2)) {
+      cur ^= 1;
+      continue;
+    }
     if (fuse != nullptr && it == hp->ns_steps - 1) {
       // the last X' = B' X updates the parameters instead of being stored: the
       // finish pass's arithmetic (muon_update_element) on the same bf16 values
@@ -877,13 +909,13 @@ int finish(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
 // when the shape allows (can_fuse_update), else the finish pass after the chain.
 int newton_schulz_finish(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols,
                          const morph_muon_hp* hp, void* workspace, size_t workspace_bytes,
-                         void* stream) {
+                         void* stream, Part part = Part::kAll) {
   Bufs W;
   int rc = setup(mats, count, rows, cols, hp, workspace, workspace_bytes, true, false, &W);
   if (rc || count == 0) return rc;
   if (hp->ns_steps >= 1 && (takes_small(W.L, hp) || can_fuse_update(mats, count, W.L)))
-    return newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, mats);
-  rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream);
+    return newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, mats, part);
+  rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, nullptr, part);
   if (!rc) rc = finish(mats, count, rows, cols, hp, workspace, workspace_bytes, false, stream);
   return rc;
 }
@@ -925,6 +957,21 @@ extern "C" int morph_muon_newton_schulz_finish(const morph_muon_matrix* mats, in
                                                const morph_muon_hp* hp, void* workspace,
                                                size_t workspace_bytes, void* stream) {
   return newton_schulz_finish(mats, count, rows, cols, hp, workspace, workspace_bytes, stream);
+}
+
+extern "C" int morph_muon_newton_schulz_ahead(int count, int64_t rows, int64_t cols,
+                                              const morph_muon_hp* hp, void* workspace,
+                                              size_t workspace_bytes, void* stream) {
+  return newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, nullptr,
+                       Part::kAhead);
+}
+
+extern "C" int morph_muon_newton_schulz_finish_rest(const morph_muon_matrix* mats, int count,
+                                                    int64_t rows, int64_t cols,
+                                                    const morph_muon_hp* hp, void* workspace,
+                                                    size_t workspace_bytes, void* stream) {
+  return newton_schulz_finish(mats, count, rows, cols, hp, workspace, workspace_bytes, stream,
+                              Part::kRest);
 }
 
 extern "C" int morph_muon_step(const morph_muon_matrix* mats, int count, int64_t rows,

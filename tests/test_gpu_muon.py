@@ -636,6 +636,59 @@ def test_update_in_the_last_product_equals_the_finish_pass(rows, cols, steps):
         assert not torch.equal(results[0][0][i].cpu(), p0[i])  # the update happened
 
 
+@pytest.mark.parametrize("rows,cols,steps", [(256, 512, 5), (512, 256, 1), (192, 320, 5),
+                                             (1536, 3072, 5), (96, 200, 5), (256, 256, 0)])
+def test_chain_in_two_calls_equals_one(rows, cols, steps):
+    """morph_muon_newton_schulz_ahead writes no parameter; with _finish_rest behind it the bits
+    are those of newton_schulz_finish (with padding and without, a chain that the first
+    call runs to its last product, one whose first product is cover enough, the
+    one-launch chain, no iterations), and a step dropped in between leaves nothing behind."""
+    import ctypes
+    from morph_amd import _lib
+    L = _lib.lib()
+    gen = torch.Generator().manual_seed(rows + cols + steps)
+    shapes = [(rows, cols), (cols, rows)]
+    p0 = [torch.randn(s, generator=gen) * .02 for s in shapes]
+    g = [(torch.randn(s, generator=gen) * 1e-3).to(DEV) for s in shapes]
+    bad = [x.clone() for x in g]
+    bad[0][1, 2] = float("nan")
+    hp = muon._step_hp(rows, cols, .02, .01, steps)
+    hpp = ctypes.byref(hp)
+    ws = torch.zeros(L.morph_muon_workspace_bytes(rows, cols, 2), dtype=torch.uint8, device=DEV)
+    wsp, wsn, sh = ctypes.c_void_p(ws.data_ptr()), ws.numel(), _lib.stream_handle()
+    results = []
+    for split in (False, True):
+        p, m = [t.to(DEV) for t in p0], [torch.zeros(s, device=DEV) for s in shapes]
+        drop = [torch.zeros(s, device=DEV) for s in shapes]
+
+        def descriptors(grads, momenta):
+            arr = (_lib.MuonMatrix * 2)()
+            for i in range(2):
+                arr[i].grad, arr[i].momentum = grads[i].data_ptr(), momenta[i].data_ptr()
+                arr[i].param, arr[i].transposed = p[i].data_ptr(), int(shapes[i] != (rows, cols))
+            return arr
+
+        if split:
+            arr = descriptors(bad, drop)
+            _lib.check(L.morph_muon_prepare(arr, 2, rows, cols, hpp, 0, wsp, wsn, None, sh))
+            _lib.check(L.morph_muon_newton_schulz_ahead(2, rows, cols, hpp, wsp, wsn, sh))
+        arr = descriptors(g, m)
+        _lib.check(L.morph_muon_prepare(arr, 2, rows, cols, hpp, 0, wsp, wsn, None, sh))
+        if split:
+            _lib.check(L.morph_muon_newton_schulz_ahead(2, rows, cols, hpp, wsp, wsn, sh))
+            torch.cuda.synchronize()
+            assert all(torch.equal(a.cpu(), b) for a, b in zip(p, p0))
+            _lib.check(L.morph_muon_newton_schulz_finish_rest(arr, 2, rows, cols, hpp, wsp, wsn, sh))
+        else:
+            _lib.check(L.morph_muon_newton_schulz_finish(arr, 2, rows, cols, hpp, wsp, wsn, sh))
+        torch.cuda.synchronize()
+        results.append((p, m))
+    for i in range(2):
+        assert torch.equal(results[0][0][i], results[1][0][i]), i
+        assert torch.equal(results[0][1][i], results[1][1][i]), i
+        assert not torch.equal(results[0][0][i].cpu(), p0[i])
+
+
 def test_one_call_c_entry_equals_phased_path():
     """morph_muon_step (C convenience) == prepare + newton_schulz_finish as the Python layer runs them."""
     import ctypes
