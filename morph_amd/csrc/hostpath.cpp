@@ -88,9 +88,11 @@ class StepPlan {
       numels_[k] = desc_[k].numel;
     }
     if (n == 0) throw std::invalid_argument("a plan steps at least one tensor");
-    const at::Tensor* first = plain_tensor(PyList_GET_ITEM(params_.ptr(), present_[0]));
-    if (first == nullptr) throw std::invalid_argument("parameters must be plain tensors");
-    device_ = first->device();
+    // Any tensor will do here, a subclass's or one under a dispatch mode too: a step that
+    // cannot be taken natively is match()'s to refuse.
+    PyObject* first = PyList_GET_ITEM(params_.ptr(), present_[0]);
+    if (!THPVariable_Check(first)) throw std::invalid_argument("parameters must be tensors");
+    device_ = THPVariable_Unpack(first).device();
     type_ = grad_dtype == MORPH_DTYPE_F16    ? at::kHalf
             : grad_dtype == MORPH_DTYPE_BF16 ? at::kBFloat16
                                              : at::kFloat;

@@ -601,6 +601,41 @@ def test_native_steps_equal_python_steps(count):
         a.step([torch.zeros(2 * g.numel(), dtype=torch.half, device=DEV)[::2] for g in gs])
 
 
+class _Sub(torch.nn.Parameter):
+    pass
+
+
+@pytest.mark.parametrize("how", ["subclass", "dispatch mode"])
+def test_parameters_the_native_path_cannot_describe_step_as_others(how):
+    """Parameters of a tensor subclass, and steps under a TorchDispatchMode (a FLOP counter,
+    say), take the Python path on every step, with the bits of plain parameters' steps."""
+    import contextlib
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    gen = torch.Generator().manual_seed(17)
+    masters = [torch.randn(n, generator=gen) * .02 for n in (300, 70)]
+    grads = [[torch.randn(n, generator=gen) * 1e-3 for n in (300, 70)] for _ in range(4)]
+    runs = []
+    for odd in (True, False):
+        sub = odd and how == "subclass"
+        ps = [m.to(DEV).as_subclass(_Sub) if sub else torch.nn.Parameter(m.to(DEV)) for m in masters]
+        opt = FusedAdamW(ps, lr=1e-3)
+        for gs in grads:
+            for p, g in zip(ps, gs):
+                p.grad = g.to(DEV)
+            with Mode() if odd and not sub else contextlib.nullcontext():
+                opt.step()
+        opt.resolve()
+        runs.append([p.detach().as_subclass(torch.Tensor) for p in ps])
+    for x, y, m in zip(*runs, masters):
+        assert torch.equal(x, y) and not torch.equal(x.cpu(), m)
+
+
 @pytest.mark.parametrize("count,size", [(1, 1 << 24), (200, 1 << 16)], ids=["one", "split"])
 def test_dispatch_timer_stamps_the_adamw_launches(count, size):
     """Events stamped by the AdamW dispatch itself (hipExtLaunchKernel) time the pass: each

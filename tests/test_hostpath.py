@@ -25,8 +25,11 @@ class Case:
         for d, i in zip(self.array, self.present):
             d.numel = self.params[i].numel()
             d.out = self.exports[i].data_ptr() if exports else None
-        self.plan = _lib.hostpath().StepPlan(self.params, self.present, _lib.ctypes.addressof(self.array),
-                                             _lib.dtype_code(dtype), -1, 0, 0, 0, [0] * 5)
+        self.plan = self.make_plan()
+
+    def make_plan(self):
+        return _lib.hostpath().StepPlan(self.params, self.present, _lib.ctypes.addressof(self.array),
+                                        _lib.dtype_code(self.dtype), -1, 0, 0, 0, [0] * 5)
 
     def grads(self):
         return [torch.ones(s, dtype=self.dtype) if i in self.present else None
@@ -108,6 +111,35 @@ def test_other_views_with_the_same_layout_match():
     gs[0] = torch.ones(24)
     gs[3] = torch.ones(10)[1:]
     assert c.match(gs) and c.array[2].grad == gs[3].data_ptr()
+
+
+class Sub(torch.nn.Parameter):
+    pass
+
+
+def test_a_plan_over_subclass_parameters_refuses_their_own_gradients():
+    """Parameters of a tensor subclass step on the Python path: no plan error on the way."""
+    c = Case()
+    c.params[0] = c.groups[0]["params"][0] = torch.zeros(4, 6).as_subclass(Sub)
+    c.plan = c.make_plan()
+    for i in c.present:
+        c.params[i].grad = torch.ones(SHAPES[i])
+    assert not c.match()
+
+
+def test_a_plan_made_under_a_dispatch_mode_waits_for_its_end():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    c = Case()
+    gs = c.grads()
+    with Mode():
+        c.plan = c.make_plan()
+        assert not c.match(gs)
+    assert c.match(gs)
 
 
 def test_bad_plans_raise():
