@@ -6,10 +6,11 @@
 // beside 9 and 10.5 us of kernels; here 12.5 and 25.8 us.
 //
 // StepPlan belongs to one descriptor batch (kernels.AdamwBatch) and keeps no check from one
-// step to the next: match() looks at every parameter and gradient again and says no on
-// anything that is not exactly what the batch was built for (another parameter list, a
-// gradient missing or new, another type, device, size or layout, a tensor subclass, other
-// export buffers); the caller then takes the Python path, which rebuilds or raises.
+// step to the next: match() looks at every parameter, both its moments and its gradient again
+// and says no on anything that is not exactly what the batch was built for (another parameter
+// list, a parameter or a moment that lies elsewhere, a gradient missing or new, another type,
+// device, size or layout, a tensor subclass, other export buffers); the caller then takes the
+// Python path, which rebuilds or raises.
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
@@ -23,11 +24,22 @@ namespace py = pybind11;
 
 namespace {
 
+// at::isTensorSubclassLike without its question for a dispatch mode, which match() asks once.
+bool plain(const at::Tensor& t) {
+  return (t.key_set() & at::kTensorSubclassLike).empty() && t.has_storage();
+}
+
 const at::Tensor* plain_tensor(PyObject* o) {
   if (o == nullptr || !THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
-  if (!t.defined() || at::isTensorSubclassLike(t) || !t.has_storage()) return nullptr;
-  return &t;
+  return t.defined() && plain(t) ? &t : nullptr;
+}
+
+// Whether o is still the n floats at `address` that a descriptor points at.
+bool still_at(PyObject* o, const void* address, int64_t n) {
+  const at::Tensor* t = plain_tensor(o);
+  return t != nullptr && t->numel() == n && t->scalar_type() == at::kFloat && t->is_contiguous() &&
+         t->const_data_ptr() == address;
 }
 
 // A list's or tuple's items, borrowed; false for anything else.
@@ -98,13 +110,15 @@ class StepPlan {
                                              : at::kFloat;
   }
 
-  // Whether this step's parameters, gradients and export buffers are what the batch was
-  // built for; if so the descriptors now hold the gradients' addresses and the plan holds
+  // Whether this step's parameters, moments, gradients and export buffers are what the batch
+  // was built for; if so the descriptors now hold the gradients' addresses and the plan holds
   // the gradients (until the next match).  grads: None (each parameter's .grad), or a
-  // list or tuple with an entry (or None) per parameter.
-  bool match(py::handle groups, py::handle grads, py::handle exports) {
+  // list or tuple with an entry (or None) per parameter.  state: the optimizer's, {parameter:
+  // {exp_avg, exp_avg_sq, ..}} in the parameters' order.
+  bool match(py::handle groups, py::handle grads, py::handle exports, py::handle state) {
     const Items gs(groups.ptr()), outs(exports.ptr());
-    if (!gs.ok || !outs.ok) return false;
+    if (!gs.ok || !outs.ok || !PyDict_Check(state.ptr())) return false;
+    if (c10::impl::dispatch_mode_enabled()) return false;
     const bool own = grads.is_none();
     const Items given(own ? groups.ptr() : grads.ptr());
     const Py_ssize_t total = PyList_GET_SIZE(params_.ptr());
@@ -112,7 +126,7 @@ class StepPlan {
     if (outs.n != 0 && outs.n != total) return false;
     std::vector<at::Tensor> held;
     held.reserve(present_.size());
-    Py_ssize_t i = 0;
+    Py_ssize_t i = 0, in_state = 0;
     size_t k = 0;
     for (Py_ssize_t g = 0; g < gs.n; ++g) {
       PyObject* group = gs.at(g);
@@ -123,14 +137,16 @@ class StepPlan {
       for (Py_ssize_t j = 0; j < PyList_GET_SIZE(list); ++j, ++i) {
         PyObject* po = PyList_GET_ITEM(list, j);
         if (i >= total || po != PyList_GET_ITEM(params_.ptr(), i)) return false;
+        PyObject *owner = nullptr, *moments = nullptr;  // borrowed
+        if (!PyDict_Next(state.ptr(), &in_state, &owner, &moments) || owner != po) return false;
         const bool want = k < present_.size() && present_[k] == i;
         at::Tensor grad;
         if (own) {
           const at::Tensor* p = plain_tensor(po);
           if (p == nullptr) return false;
-          grad = p->grad();
+          grad = p->unsafeGetTensorImpl()->grad();
           if (grad.defined() != want) return false;
-          if (want && (at::isTensorSubclassLike(grad) || !grad.has_storage())) return false;
+          if (want && !plain(grad)) return false;
         } else {
           PyObject* go = given.at(i);
           if ((go == Py_None) == want) return false;
@@ -141,6 +157,13 @@ class StepPlan {
           }
         }
         if (!want) continue;
+        static PyObject* const first = PyUnicode_InternFromString("exp_avg");
+        static PyObject* const second = PyUnicode_InternFromString("exp_avg_sq");
+        const morph_adamw_tensor& d = desc_[k];
+        if (!PyDict_Check(moments) || !still_at(po, d.param, d.numel) ||
+            !still_at(PyDict_GetItemWithError(moments, first), d.exp_avg, d.numel) ||
+            !still_at(PyDict_GetItemWithError(moments, second), d.exp_avg_sq, d.numel))
+          return false;
         if (grad.layout() != at::kStrided || grad.device() != device_ ||
             grad.scalar_type() != type_ || grad.numel() != numels_[k] || !grad.is_contiguous())
           return false;

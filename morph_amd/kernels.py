@@ -189,6 +189,14 @@ class AdamwBatch:
                 "morph_nonfinite_or_multi", "morph_nonfinite_or_close", "morph_adamw_multi_dev",
                 "morph_nonfinite_table", "morph_adamw_table_dev")])
 
+    def used_on(self, stream):
+        """Keep the batch's masters, moments and exports for the work queued on `stream`."""
+        if stream != torch.cuda.current_stream(self._device):
+            for tensors in self._keep:
+                for t in tensors:
+                    if t is not None and t.is_cuda:
+                        t.record_stream(stream)
+
     def handed_over(self, stream):
         """A StepPlan holds the gradients from here on; the table is read on `stream`."""
         self._grads = None

@@ -244,6 +244,18 @@ class FusedAdamW:
             self._tables[key] = BiasTables(key[0], key[1], self.device)
         return self._tables[key]
 
+    def _places(self, present):
+        """Where the listed masters and moments lie: a caller may move a parameter (p.data) or
+        replace a moment in self.state between steps."""
+        masters = [self._dev[i] for i in present]
+        states = [self.state[p] for p in self._listed(present)]
+        return (tuple((p.data_ptr(), p.numel(), p.is_contiguous()) for p in masters),
+                tuple((s["exp_avg"].data_ptr(), s["exp_avg_sq"].data_ptr()) for s in states))
+
+    def _listed(self, present):
+        flat = self._flat()
+        return [flat[i][1] for i in present]
+
     def _prepare(self, grads, present):
         """Descriptor batch, clock list and parameter groups for this set of tensors."""
         flat = self._flat()
@@ -252,10 +264,14 @@ class FusedAdamW:
         if self._plan is not None:
             self._plan.release()
         key = (tuple(present), tuple(grads[i].dtype for i in present),
-               tuple(e.data_ptr() for e in self.exports) if self.exports else None)
+               tuple(e.data_ptr() for e in self.exports) if self.exports else None,
+               self._places(present))
         ptrs = tuple(grads[i].data_ptr() for i in present)
         if key != self._cache_key:
-            ps = [flat[i][1] for i in present]
+            ps = self._listed(present)
+            if self._cache is not None and self._pending is not None:
+                # tensors that only the old batch still holds may be in use there
+                self._cache[0].used_on(self._pending[2])
             batch = kernels.AdamwBatch(
                 [self._dev[i] for i in present], [self.state[p]["exp_avg"] for p in ps],
                 [self.state[p]["exp_avg_sq"] for p in ps], [grads[i] for i in present],
@@ -323,7 +339,7 @@ class FusedAdamW:
         # the batch's descriptors are up to date and the launches go out natively
         if (self._plan is not None and self._plan_key is self._cache_key
                 and self.kernel_timer is None and self.dispatch_timer is None
-                and self._plan.match(self.param_groups, grads, self.exports)):
+                and self._plan.match(self.param_groups, grads, self.exports, self.state)):
             self._cache[2] = None  # the descriptors' addresses are the plan's now
             return self._enqueue(None, None, stream, checked, planned=True)
         return self._step(grads, stream, checked)
@@ -417,7 +433,8 @@ class FusedAdamW:
         flat = self._flat()
         key = (tuple(present), tuple(grads[i].dtype for i in present),
                tuple(grads[i].data_ptr() for i in present),
-               tuple(e.data_ptr() for e in self.exports) if self.exports else None)
+               tuple(e.data_ptr() for e in self.exports) if self.exports else None,
+               self._places(present))
         if self._chunk_cache is not None and self._chunk_cache[0] == key:
             return self._chunk_cache[1]
         batches = []

@@ -601,6 +601,68 @@ def test_native_steps_equal_python_steps(count):
         a.step([torch.zeros(2 * g.numel(), dtype=torch.half, device=DEV)[::2] for g in gs])
 
 
+@pytest.mark.parametrize("masters_on", ["gpu", "gpu, Python path", "cpu"])
+def test_moved_parameters_and_replaced_moments_are_the_ones_stepped(masters_on):
+    """Between two steps of the same tensors a caller moves a parameter (p.data, CPU masters too)
+    or puts other moments into opt.state: the next step reads and updates what is there now, as
+    an optimizer that starts from those values does, and leaves the old storage alone."""
+    gen = torch.Generator().manual_seed(23)
+    n = 3000
+    start = [torch.randn(n, generator=gen) * .02 for _ in range(3)]
+    grads = [[torch.randn(n, generator=gen) * 1e-3 for _ in start] for _ in range(8)]
+    host = masters_on == "cpu"
+    put = (lambda t: t.clone()) if host else (lambda t: t.to(DEV))
+    ps = [torch.nn.Parameter(put(t)) for t in start]
+    opt = FusedAdamW(ps, lr=1e-3)
+    steps = []
+
+    def step(gs):
+        if masters_on == "gpu, Python path":
+            opt.kernel_timer = []
+        opt.step([g.to(DEV) for g in gs])
+        steps.append(opt._cache[2] is None)
+
+    ref_w, ref_m, ref_v = ([t.numpy().copy() for t in start], [np.zeros(n, np.float32) for _ in start],
+                           [np.zeros(n, np.float32) for _ in start])
+    from oracle import reference as R
+
+    def ref(gs, t):
+        for i, g in enumerate(gs):
+            R.adamw(g.numpy(), ref_w[i], ref_m[i], ref_v[i], R.torch_adamw_hp(1e-3, .9, .999, 1e-8, .01, t))
+
+    t = 0
+    for k in range(3):
+        t += 1
+        step(grads[k]), ref(grads[k], t)
+    old = ps[0].data
+    opt.resolve()
+    was = old.clone()
+    moved = torch.randn(n, generator=gen) * .02
+    ps[0].data = put(moved)
+    ref_w[0] = moved.numpy().copy()
+    for k in (3, 4, 5):
+        t += 1
+        step(grads[k]), ref(grads[k], t)
+    opt.resolve()
+    assert torch.equal(old, was)
+    first, second = torch.randn(n, generator=gen) * 1e-4, torch.rand(n, generator=gen) * 1e-6
+    opt.state[ps[1]]["exp_avg"] = first.to(DEV)
+    opt.state[ps[2]]["exp_avg_sq"] = second.to(DEV)
+    ref_m[1], ref_v[2] = first.numpy().copy(), second.numpy().copy()
+    for k in (6, 7):
+        t += 1
+        step(grads[k]), ref(grads[k], t)
+    opt.resolve()
+    if masters_on == "gpu":
+        assert steps == [False, False, True] * 2 + [False, False]
+    else:
+        assert not any(steps)
+    for i, p in enumerate(ps):
+        assert_same_bits(p.detach().cpu().numpy(), ref_w[i], f"master {i}")
+        assert_same_bits(opt.state[p]["exp_avg"].cpu().numpy(), ref_m[i], f"exp_avg {i}")
+        assert_same_bits(opt.state[p]["exp_avg_sq"].cpu().numpy(), ref_v[i], f"exp_avg_sq {i}")
+
+
 class _Sub(torch.nn.Parameter):
     pass
 

@@ -19,11 +19,15 @@ class Case:
         self.params = [torch.nn.Parameter(torch.zeros(s)) for s in SHAPES]
         self.groups = [dict(params=self.params[:2], lr=1.0), dict(params=self.params[2:], lr=2.0)]
         self.present = [0, 2, 3]
+        self.state = {p: dict(step=0, exp_avg=torch.zeros_like(p.data), exp_avg_sq=torch.zeros_like(p.data))
+                      for p in self.params}
         self.dtype = dtype
         self.exports = [torch.zeros(s, dtype=torch.float16) for s in SHAPES] if exports else []
         self.array = (_lib.AdamwTensor * 3)()
         for d, i in zip(self.array, self.present):
-            d.numel = self.params[i].numel()
+            p = self.params[i]
+            d.numel, d.param = p.numel(), p.data_ptr()
+            d.exp_avg, d.exp_avg_sq = (self.state[p][k].data_ptr() for k in ("exp_avg", "exp_avg_sq"))
             d.out = self.exports[i].data_ptr() if exports else None
         self.plan = self.make_plan()
 
@@ -37,7 +41,7 @@ class Case:
 
     def match(self, grads=None):
         before = [d.grad for d in self.array]
-        ok = self.plan.match(self.groups, grads, self.exports)
+        ok = self.plan.match(self.groups, grads, self.exports, self.state)
         if not ok:
             assert [d.grad for d in self.array] == before  # a refusal writes nothing
         return ok
@@ -86,7 +90,20 @@ def test_the_parameters_own_gradients():
     lambda c, g: c.groups[1].__setitem__("params", tuple(c.params[2:])),
     lambda c, g: c.exports.__setitem__(3, torch.zeros(3, 3, dtype=torch.float16)),
     lambda c, g: c.exports.clear(), lambda c, g: c.exports.pop(),
-], ids=range(22))
+    # a parameter that lies elsewhere, or is another size or layout where it lay
+    lambda c, g: setattr(c.params[0], "data", torch.zeros(4, 6)),
+    lambda c, g: setattr(c.params[3], "data", c.params[3].data[:2]),
+    lambda c, g: setattr(c.params[3], "data", c.params[3].data.t()),
+    # a moment replaced, moved, or gone
+    lambda c, g: c.state[c.params[0]].__setitem__("exp_avg", torch.zeros(4, 6)),
+    lambda c, g: c.state[c.params[3]].__setitem__("exp_avg_sq", torch.zeros(3, 3)),
+    lambda c, g: setattr(c.state[c.params[3]]["exp_avg"], "data", torch.zeros(3, 3)),
+    lambda c, g: c.state[c.params[3]].pop("exp_avg_sq"),
+    lambda c, g: c.state.__setitem__(c.params[0], {k: v for k, v in c.state[c.params[3]].items()}),
+    lambda c, g: c.state.pop(c.params[0]),
+    lambda c, g: setattr(c, "state", {p: c.state[p] for p in reversed(c.params)}),
+    lambda c, g: setattr(c, "state", None),
+], ids=range(33))
 def test_anything_else_is_refused(change):
     c = Case(exports=True)
     gs = c.grads()
@@ -99,7 +116,8 @@ def test_other_containers_are_refused():
     c = Case()
     gs = c.grads()
     assert not c.match(iter(gs)) and not c.match(dict(enumerate(gs)))
-    assert not c.plan.match(tuple(dict(g, params=iter(g["params"])) for g in c.groups), gs, [])
+    assert not c.plan.match(tuple(dict(g, params=iter(g["params"])) for g in c.groups), gs, [],
+                            c.state)
     assert c.match(gs)
 
 
@@ -120,7 +138,10 @@ class Sub(torch.nn.Parameter):
 def test_a_plan_over_subclass_parameters_refuses_their_own_gradients():
     """Parameters of a tensor subclass step on the Python path: no plan error on the way."""
     c = Case()
-    c.params[0] = c.groups[0]["params"][0] = torch.zeros(4, 6).as_subclass(Sub)
+    sub = torch.zeros(4, 6).as_subclass(Sub)
+    c.state = {sub if p is c.params[0] else p: s for p, s in c.state.items()}
+    c.params[0] = c.groups[0]["params"][0] = sub
+    c.array[0].param = sub.data_ptr()
     c.plan = c.make_plan()
     for i in c.present:
         c.params[i].grad = torch.ones(SHAPES[i])
