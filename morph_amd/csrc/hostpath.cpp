@@ -190,9 +190,11 @@ class StepPlan {
 
   // The step's launches on `stream` after match(): the detector (unless `checked`; with the
   // previous step's close when prev_list is not 0), then AdamW.  The status of the first
-  // that failed, or 0.
+  // that failed, or 0.  The GIL is released meanwhile, as around every other call of the
+  // library: a launch waits when the queue is full.
   int launch(uint64_t stream, int slot, bool checked, uint64_t prev_list, int n_prev,
              uint64_t hps, uint64_t scheds, int n_hp) {
+    const py::gil_scoped_release nogil;
     void* s = reinterpret_cast<void*>(stream);
     const int32_t* prev = reinterpret_cast<const int32_t*>(prev_list);
     const int count = (int)present_.size();

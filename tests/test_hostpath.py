@@ -2,8 +2,13 @@
 
 match() may say yes only when the Python path would step exactly the batch's tensors with
 these gradients: everything else is its refusal, after which the Python path rebuilds the
-batch or raises.  No launch here: the entry points' addresses are never called.
+batch or raises.  No entry point of the library is called: the plans have none, or the test's.
 """
+import ctypes
+import subprocess
+import threading
+import time
+
 import pytest
 import torch
 
@@ -31,9 +36,9 @@ class Case:
             d.out = self.exports[i].data_ptr() if exports else None
         self.plan = self.make_plan()
 
-    def make_plan(self):
+    def make_plan(self, entries=(0,) * 5):
         return _lib.hostpath().StepPlan(self.params, self.present, _lib.ctypes.addressof(self.array),
-                                        _lib.dtype_code(self.dtype), -1, 0, 0, 0, [0] * 5)
+                                        _lib.dtype_code(self.dtype), -1, 0, 0, 0, list(entries))
 
     def grads(self):
         return [torch.ones(s, dtype=self.dtype) if i in self.present else None
@@ -161,6 +166,38 @@ def test_a_plan_made_under_a_dispatch_mode_waits_for_its_end():
         c.plan = c.make_plan()
         assert not c.match(gs)
     assert c.match(gs)
+
+
+def test_launches_release_the_gil(tmp_path):
+    """Other Python threads run while a launch waits (for room in a full queue, say): the entry
+    points here wait, two seconds at most, for a word that another thread writes."""
+    src = tmp_path / "entries.c"
+    src.write_text("""
+        #include <time.h>
+        volatile int started, seen;
+        int entry(void) {
+          const time_t end = time(0) + 2;
+          started = 1;
+          while (!seen && time(0) <= end) { const struct timespec t = {0, 1000000}; nanosleep(&t, 0); }
+          return seen ? 0 : -1;
+        }""")
+    lib = tmp_path / "entries.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    entries = ctypes.CDLL(str(lib))
+    c = Case()
+    c.plan = c.make_plan([ctypes.cast(entries.entry, ctypes.c_void_p).value] * 5)
+    assert c.match(c.grads())
+    started, seen = (ctypes.c_int.in_dll(entries, n) for n in ("started", "seen"))
+
+    def answer():
+        while not started.value:
+            time.sleep(1e-3)
+        seen.value = 1
+
+    thread = threading.Thread(target=answer, daemon=True)
+    thread.start()
+    assert c.plan.launch(0, 0, False, 0, 0, 0, 0, 0) == 0
+    thread.join()
 
 
 def test_bad_plans_raise():
