@@ -199,6 +199,7 @@ class StepPlan {
     const int32_t* prev = reinterpret_cast<const int32_t*>(prev_list);
     const int count = (int)present_.size();
     int rc = MORPH_OK;
+    closed_ = false;
     if (!checked) {
       if (table_ != nullptr)
         rc = fn_.nonfinite_table(table_, desc_, count, grad_dtype_, state_, slot, clocks_, prev,
@@ -211,6 +212,7 @@ class StepPlan {
                                     &state_->found_inf[slot], s);
       if (rc != MORPH_OK) return rc;
     }
+    closed_ = true;
     const morph_adamw_hp* h = reinterpret_cast<const morph_adamw_hp*>(hps);
     const morph_adamw_sched* c = reinterpret_cast<const morph_adamw_sched*>(scheds);
     if (table_ != nullptr)
@@ -219,6 +221,9 @@ class StepPlan {
     return fn_.adamw_multi_dev(desc_, count, grad_dtype_, out_dtype_, h, c, n_hp, clocks_, state_,
                                slot, nullptr, nullptr, s);
   }
+
+  // Whether the last launch() got past the detector, which carries the previous step's close.
+  bool closed() const { return closed_; }
 
  private:
   py::list params_;
@@ -232,6 +237,7 @@ class StepPlan {
   std::vector<int64_t> numels_;
   std::vector<const void*> ptrs_;
   std::vector<at::Tensor> held_;
+  bool closed_ = false;
   at::Device device_{at::kCPU};
   at::ScalarType type_;
 };
@@ -244,5 +250,6 @@ PYBIND11_MODULE(_hostpath, m) {
                     std::vector<uint64_t>>())
       .def("match", &StepPlan::match)
       .def("release", &StepPlan::release)
+      .def("closed", &StepPlan::closed)
       .def("launch", &StepPlan::launch);
 }

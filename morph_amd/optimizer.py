@@ -494,11 +494,13 @@ class FusedAdamW:
         if planned:
             prev = self._pending[1] if self._pending is not None else None
             batch.handed_over(s)
-            kernels.check(self._plan.launch(
+            status = self._plan.launch(
                 s.cuda_stream, slot, checked, prev.data_ptr() if prev is not None else 0,
                 prev.numel() if prev is not None else 0, ctypes.addressof(hps),
-                ctypes.addressof(scheds), len(hps)))
-            self._pending = None
+                ctypes.addressof(scheds), len(hps))
+            if status == 0 or self._plan.closed():
+                self._pending = None
+            kernels.check(status)
         elif not checked:
             prev = self._pending[1] if self._pending is not None else None
             batch.detect([grads[i] for i in present], ctl.state, slot, ctl.clocks, prev, s)

@@ -601,6 +601,40 @@ def test_native_steps_equal_python_steps(count):
         a.step([torch.zeros(2 * g.numel(), dtype=torch.half, device=DEV)[::2] for g in gs])
 
 
+def test_a_failed_launch_closes_the_previous_step_once(monkeypatch):
+    """The AdamW launch of a native step fails (the entry point refuses) behind the detector that
+    closed the step before it: the error is raised, and the steps that follow count that close
+    once and apply as if the failed step had not been asked for."""
+    import ctypes
+
+    from morph_amd import _lib
+    refuse = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: -1)
+    w0 = torch.randn(1000, generator=torch.Generator().manual_seed(3)) * .02
+    grads = [torch.randn(1000, generator=torch.Generator().manual_seed(40 + k)).to(DEV) for k in range(5)]
+    runs = []
+    for fails in (True, False):
+        w = w0.to(DEV)
+        opt = FusedAdamW([w], lr=1e-3, loss_scale=DynamicLossScale(1024.0))
+        for g in grads[:3]:
+            opt.step([g])
+        if fails:
+            real, batch = opt._plan, opt._cache[0]
+            address = _lib.entry_address
+            monkeypatch.setattr(_lib, "entry_address", lambda name: ctypes.cast(
+                refuse, ctypes.c_void_p).value if name == "morph_adamw_multi_dev" else address(name))
+            opt._plan = batch.step_plan([w], [0], opt._ctl.clocks, opt._ctl.state)
+            with pytest.raises(_lib.MorphError):
+                opt.step([grads[3]])
+            opt._plan = real
+        for g in grads[3:]:
+            opt.step([g])
+        opt.resolve()
+        runs.append((w, opt.state[w], opt.applied_steps, opt.loss_scale.state_dict()))
+    (w, st, applied, scaler), (rw, rst, rapplied, rscaler) = runs
+    assert st["step"] == rst["step"] == 5 and applied == rapplied == 5 and scaler == rscaler
+    assert torch.equal(w, rw) and torch.equal(st["exp_avg_sq"], rst["exp_avg_sq"])
+
+
 @pytest.mark.parametrize("masters_on", ["gpu", "gpu, Python path", "cpu"])
 def test_moved_parameters_and_replaced_moments_are_the_ones_stepped(masters_on):
     """Between two steps of the same tensors a caller moves a parameter (p.data, CPU masters too)

@@ -200,6 +200,19 @@ def test_launches_release_the_gil(tmp_path):
     thread.join()
 
 
+@pytest.mark.parametrize("detector,adamw,closed", [(-1, 0, False), (0, -1, True), (0, 0, True)])
+def test_launch_says_whether_the_detector_went_out(detector, adamw, closed):
+    """The detector's launch carries the previous step's close: a step whose AdamW launch fails
+    behind it has closed that step."""
+    made = [ctypes.CFUNCTYPE(ctypes.c_int)(lambda rc=rc: rc) for rc in (detector, adamw)]
+    det, upd = (ctypes.cast(f, ctypes.c_void_p).value for f in made)
+    c = Case()
+    c.plan = c.make_plan([det, det, upd, det, upd])
+    assert c.match(c.grads()) and not c.plan.closed()
+    assert c.plan.launch(0, 0, False, 0, 0, 0, 0, 0) == (detector or adamw)
+    assert c.plan.closed() == closed
+
+
 def test_bad_plans_raise():
     p = [torch.zeros(3)]
     make = lambda present, entries=5: _lib.hostpath().StepPlan(  # noqa: E731
