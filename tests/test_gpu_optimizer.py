@@ -618,11 +618,11 @@ def test_a_failed_launch_closes_the_previous_step_once(monkeypatch):
         for g in grads[:3]:
             opt.step([g])
         if fails:
-            real, batch = opt._plan, opt._cache[0]
-            address = _lib.entry_address
-            monkeypatch.setattr(_lib, "entry_address", lambda name: ctypes.cast(
-                refuse, ctypes.c_void_p).value if name == "morph_adamw_multi_dev" else address(name))
-            opt._plan = batch.step_plan([w], [0], opt._ctl.clocks, opt._ctl.state)
+            real, address = opt._plan, _lib.entry_address
+            with monkeypatch.context() as patch:
+                patch.setattr(_lib, "entry_address", lambda name: ctypes.cast(
+                    refuse, ctypes.c_void_p).value if name == "morph_adamw_multi_dev" else address(name))
+                opt._plan = opt._cache[0].step_plan([w], [0], opt._ctl.clocks, opt._ctl.state)
             with pytest.raises(_lib.MorphError):
                 opt.step([grads[3]])
             opt._plan = real
