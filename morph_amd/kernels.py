@@ -108,14 +108,31 @@ class AdamwBatch:
             keep.append((p, m, v, o))
         self._keep = keep  # the tensors must outlive the descriptors
         self._grads = list(grads)
-        self._table = self._device_table() if n > _lib.ADAMW_LAUNCH_TENSORS else None
+        self._table = None
         self._grad_dtype = grads[0].dtype if n else None
         self._numels = [p.numel() for p in params]
         self._device = params[0].device if n else None
 
+    def make_table(self, kept):
+        """Let detect(), launch_dev() and step_plan() run over a descriptor table in device memory
+        (adamw_table.h), for a group of more tensors than the kernel arguments hold.  Making it
+        costs host time by the elements (4 bytes per 256, filled here) and a copy that waits for
+        the current stream, so it is left to a caller that steps the same tensors again.  kept:
+        this is such a step already; else it might be the only one, and only a table that is
+        soon made is.
+
+        Measured, FP32 gradients, first step of a new group with and without it: 64 tensors of
+        65536 elements 1.70 and 1.57 ms, of 2^20 1.96 and 1.85 ms, 60 of 18874368 11.8 and
+        7.5 ms; 100 of 16384: within the runs.  A later step: 16 and 24 us for 100 of 16384,
+        245 and 275 us for 200 of 2^18, 1367 and 1391 us for 64 of 2^22 (2^20 blocks); 60 of
+        18874368 5.77 ms with both."""
+        elements = sum(self._numels)
+        if self._table is None and self.count > _lib.ADAMW_LAUNCH_TENSORS and (
+                elements <= self.count << 14 or (kept and elements <= 1 << 28)):
+            self._table = self._device_table()
+
     def _device_table(self):
-        """The descriptors in device memory (morph_adamw_table_fill), for the one-launch forms
-        of groups with more tensors than the kernel arguments hold; None outside its limits."""
+        """The descriptors in device memory (morph_adamw_table_fill); None outside its limits."""
         if (self.n_hp > _lib.ADAMW_TABLE_SETS
                 or any(d.numel > _lib.ADAMW_TABLE_NUMEL for d in self.array)
                 or any(d.clock_index < 0 for d in self.array)):
@@ -130,9 +147,10 @@ class AdamwBatch:
         return host.to(self._keep[0][0].device)
 
     def _use_table(self, stream):
-        """The table, kept for work enqueued on another stream than the one that was current
-        when it was allocated."""
-        if stream is not None and stream != self._table_stream:
+        """The table, kept for work enqueued on another stream (None: the current one) than the
+        one that was current when it was allocated."""
+        stream = stream or torch.cuda.current_stream(self._device)
+        if stream != self._table_stream:
             self._table.record_stream(stream)
         return _ptr(self._table)
 

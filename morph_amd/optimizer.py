@@ -277,6 +277,7 @@ class FusedAdamW:
                 [self.state[p]["exp_avg_sq"] for p in ps], [grads[i] for i in present],
                 [self.exports[i] for i in present] if self.exports else None,
                 hp_index=[hp_of[flat[i][0]] for i in present], clock_index=list(present))
+            batch.make_table(kept=False)
             clock_list = torch.tensor(present, dtype=torch.int32).to(self.device)
             self._cache = [batch, clock_list, ptrs, groups]
             self._cache_key = key
@@ -284,6 +285,8 @@ class FusedAdamW:
             return batch, clock_list, groups
         if self._plan is None and self._staging is None:
             # the same tensors again: their next steps can take the native path
+            if not torch.cuda.is_current_stream_capturing():
+                self._cache[0].make_table(kept=True)
             self._plan = self._cache[0].step_plan([p for _, p in flat], present, self._ctl.clocks,
                                                   self._ctl.state)
             self._plan_key = self._cache_key

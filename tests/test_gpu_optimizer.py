@@ -548,6 +548,91 @@ def test_descriptor_table_equals_kernel_argument_launches(monkeypatch, dtype, ex
         a.step([strided] + [torch.zeros(n, dtype=dtype, device=DEV) for n in sizes[1:]])
 
 
+def _group(count, size, seed=5):
+    gen = torch.Generator().manual_seed(seed)
+    return ([torch.randn(size, generator=gen) * .02 for _ in range(count)],
+            [(torch.randn(size, generator=gen) * 1e-3).to(DEV) for _ in range(count)])
+
+
+@pytest.mark.parametrize("size", [16384, 16385])
+def test_large_tensors_get_their_table_when_they_are_stepped_again(monkeypatch, size):
+    """Up to 16384 elements a tensor the table is made with the batch; above, at the second step
+    of the same tensors, and a loop that alternates between two sets of gradients makes none.
+    The same bytes without any."""
+    from morph_amd import kernels
+    masters, grads = _group(49, size)
+    other = [None] + grads[1:-1] + [None]  # 47 tensors: never a table
+    fewer = [None] + _group(50, size)[1]
+    made, runs = [], []
+    for table in (True, False):
+        if not table:
+            monkeypatch.setattr(kernels.AdamwBatch, "_device_table", lambda self: None)
+        ps = [m.to(DEV) for m in masters + masters[:2]]
+        opt = FusedAdamW(ps, lr=1e-3)
+        for gs in (grads + [None, None], grads + [None, None], other + [None, None],
+                   fewer, grads + [None, None], fewer, fewer, fewer):
+            opt.step(gs)
+            made.append(opt._cache[0]._table is not None)
+        opt.resolve()
+        runs.append(ps)
+    small = size == 16384
+    assert made[:8] == [small, True, False, small, small, small, True, True] and not any(made[8:])
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+
+def test_many_tensors_can_be_captured_after_one_step():
+    """A step's second time over the same tensors may fall into a graph capture, which allows no
+    copy to the device: it goes without a table.  A batch of the kernels module likewise."""
+    from morph_amd import kernels
+    from morph_amd.hyper import adamw_constants
+    masters, grads = _group(49, 20000)
+    side = torch.cuda.Stream()
+    runs = []
+    for captured in (True, False):
+        ps = [m.to(DEV) for m in masters]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            opt = FusedAdamW(ps, lr=1e-3)
+            opt.step(grads)
+            side.synchronize()
+            if captured:
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    opt.step(grads)
+                    opt.step(grads)
+                assert opt._cache[0]._table is None
+            for _ in range(3):
+                if captured:
+                    graph.replay()
+                else:
+                    opt.step(grads)
+                    opt.step(grads)
+                side.synchronize()
+            opt.resolve()
+        runs.append(ps + [opt.state[p]["exp_avg_sq"] for p in ps])
+        assert {opt.state[p]["step"] for p in ps} == {7}
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+    hp = adamw_constants(lr=1e-3, beta1=.9, beta2=.999, eps=1e-8, weight_decay=.01, step=1)
+    runs = []
+    for captured in (True, False):
+        ps = [m.to(DEV) for m in masters]
+        ms, vs = ([torch.zeros_like(p) for p in ps] for _ in range(2))
+        torch.cuda.synchronize()
+        if captured:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                kernels.AdamwBatch(ps, ms, vs, grads).launch([hp])
+        for _ in range(3):
+            if captured:
+                graph.replay()
+            else:
+                kernels.AdamwBatch(ps, ms, vs, grads).launch([hp])
+            torch.cuda.synchronize()
+        runs.append(ps + vs)
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+
 @pytest.mark.parametrize("count", [5, 60])
 def test_native_steps_equal_python_steps(count):
     """From a batch's second step on the launches go out natively (hostpath.cpp).  A sequence that
