@@ -153,7 +153,8 @@ class FusedAdamW:
         self._plan = None       # hostpath.StepPlan over the cached batch, from its second step on
         self._plan_key = None   # the cache key it was built for
         self._consts = None     # (hyperparameters, constants, schedules, table limit) of the groups
-        _lib.hostpath()         # a missing build fails here
+        if self._staging is None:
+            _lib.hostpath()     # a missing build fails here (CPU masters have no plan)
         self._slot = 0          # found_inf word of the next step (steps alternate)
         self._pending = None    # (slot, clock_list, stream) of a step whose close is not enqueued
         self.kernel_timer = None  # optional list: (start, end) events around each AdamW launch

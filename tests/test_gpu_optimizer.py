@@ -782,6 +782,26 @@ def test_moved_parameters_and_replaced_moments_are_the_ones_stepped(masters_on):
         assert_same_bits(opt.state[p]["exp_avg_sq"].cpu().numpy(), ref_v[i], f"exp_avg_sq {i}")
 
 
+def test_cpu_masters_need_no_host_extension(monkeypatch, tmp_path):
+    """The host extension holds the native step over device masters, and a build of it fits one
+    version of torch: without it CPU masters step as with it, and device masters say so."""
+    from morph_amd import _lib
+    w0 = torch.randn(3000, generator=torch.Generator().manual_seed(5)) * .02
+    g = torch.randn(3000, generator=torch.Generator().manual_seed(6))
+    with_it, without = w0.clone(), w0.clone()
+    opt = FusedAdamW([with_it], lr=1e-3)
+    for _ in range(3):
+        opt.step([g])
+    monkeypatch.setattr(_lib, "_hostpath", None)
+    monkeypatch.setattr(_lib, "HOSTPATH_PATH", tmp_path / "_hostpath.so")
+    opt = FusedAdamW([without], lr=1e-3)
+    for _ in range(3):
+        opt.step([g])
+    assert torch.equal(with_it, without) and not torch.equal(without, w0)
+    with pytest.raises(ImportError):
+        FusedAdamW([w0.to(DEV)])
+
+
 class _Sub(torch.nn.Parameter):
     pass
 
