@@ -533,7 +533,8 @@ int morph_muon_newton_schulz_finish(const morph_muon_matrix* mats, int count, in
  * workspace only.  _finish_rest, with the same count, rows, cols, hp and workspace,
  * enqueues what is left of the chain and the update.  Both together give the bits of
  * morph_muon_newton_schulz_finish; without _finish_rest no parameter has changed and
- * the workspace is free for another prepare.
+ * the workspace is free for another prepare behind the products, in stream order: on
+ * another stream the caller orders the two.
  */
 int morph_muon_newton_schulz_ahead(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp,
                                    void* workspace, size_t workspace_bytes, void* stream);

@@ -7,6 +7,7 @@ HybridMuonAdamW keeps the reference class's constructor, partition rule,
 step/zero_grad/state_dict/load_state_dict, with the AdamW group on FusedAdamW.
 """
 import ctypes
+import threading
 
 import torch
 from torch import nn
@@ -64,6 +65,11 @@ def gemm_nt(P, Q, D=None, alpha=1.0, beta=0.0, out=None, out_t=None, symmetric=F
     return out if batched else out[0]
 
 
+def _capturing(stream):
+    with torch.cuda.stream(stream):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class Workspaces:
     """Device workspaces of the Muon batches, one per (shape, device, batch index), each
     sized for the largest matrix count it has served.
@@ -73,10 +79,21 @@ class Workspaces:
     output, so a call on non-finite values leaves nothing behind for the next.
     Streams that used a workspace are recorded, so that a workspace replaced by a
     larger one stays allocated until their queued work is done.
+
+    One set of contents at a time: a call on another stream than the last one's waits for
+    that stream first (the last call may have been a step that its gate dropped, with its
+    first products still queued), and a call holds `lock` from its first get() to its last
+    launch, so that threads do not put their launches between each other's.  Inside a graph
+    capture nothing is waited for: replays are the caller's to order, among themselves and
+    with calls that share the workspaces.
     """
 
     def __init__(self):
         self._ws = {}
+        self.lock = threading.RLock()
+
+    def __reduce__(self):
+        return Workspaces, ()  # a copy starts with none of its own
 
     def get(self, rows, cols, count, device, index=0, stream=None):
         nbytes = lib().morph_muon_workspace_bytes(rows, cols, count)
@@ -91,8 +108,12 @@ class Workspaces:
                     entry["buf"].record_stream(s)
             with torch.cuda.stream(stream):
                 entry = dict(buf=torch.empty(nbytes, dtype=torch.uint8, device=device),
-                             streams=set())
+                             streams=set(), last=stream)
             self._ws[key] = entry
+        elif entry["last"] != stream and not _capturing(stream):
+            if not _capturing(entry["last"]):
+                stream.wait_stream(entry["last"])
+            entry["last"] = stream
         entry["streams"].add(stream)
         return entry["buf"]
 
@@ -242,12 +263,13 @@ def orthogonalize(gradients, steps=NS_STEPS, stream=None, workspaces=_WORKSPACES
         outs.append(torch.empty_like(g))
     items = [(o, g, None, None) for o, g in zip(outs, gs)]
     L, hp, sh, k = lib(), _hp(steps=steps), stream_handle(stream), 0
-    for (rows, cols), group in _by_shape(items).items():
-        for start in range(0, len(group), 64):
-            arr, count, ws = _batch(group[start:start + 64], rows, cols, stream, workspaces, k)
-            check(L.morph_muon_orthogonalize(arr, count, rows, cols, ctypes.byref(hp),
-                                             ctypes.c_void_p(ws.data_ptr()), ws.numel(), sh))
-            k += 1
+    with workspaces.lock:
+        for (rows, cols), group in _by_shape(items).items():
+            for start in range(0, len(group), 64):
+                arr, count, ws = _batch(group[start:start + 64], rows, cols, stream, workspaces, k)
+                check(L.morph_muon_orthogonalize(arr, count, rows, cols, ctypes.byref(hp),
+                                                 ctypes.c_void_p(ws.data_ptr()), ws.numel(), sh))
+                k += 1
     return outs[0] if single else outs
 
 
@@ -294,17 +316,18 @@ def muon_step(params, grads, momenta, lr, weight_decay, steps=NS_STEPS, stream=N
     """
     items = _check_items(params, grads, momenta, momenta_out)
     batches = []
-    for (rows, cols), group in _by_shape(items).items():
-        batches += _prepare(group, rows, cols, _step_hp(rows, cols, lr, weight_decay, steps),
-                            stream, workspaces, found_inf, first=len(batches))
-    ahead = probe is not None and timer is None
-    if probe is not None:
-        probe()
-    if ahead:
-        _chains_ahead(batches, stream)
-    if gate is not None:
-        gate()
-    _chains(batches, stream, timer, with_update=True, rest=ahead)
+    with workspaces.lock:
+        for (rows, cols), group in _by_shape(items).items():
+            batches += _prepare(group, rows, cols, _step_hp(rows, cols, lr, weight_decay, steps),
+                                stream, workspaces, found_inf, first=len(batches))
+        ahead = probe is not None and timer is None
+        if probe is not None:
+            probe()
+        if ahead:
+            _chains_ahead(batches, stream)
+        if gate is not None:
+            gate()
+        _chains(batches, stream, timer, with_update=True, rest=ahead)
 
 
 def _muon_grad(g, p, device):

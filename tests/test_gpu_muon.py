@@ -748,6 +748,74 @@ def test_more_than_64_matrices_run_as_several_batches():
         assert torch.equal(outs[i], muon.orthogonalize(g[i])), i
 
 
+def test_shared_workspaces_serve_streams_and_threads():
+    """The free functions' workspaces, used from two streams in turn with nothing between the
+    calls, from two threads on their own streams and from two threads on one: every result is
+    that of the call alone."""
+    import threading
+    gen = torch.Generator().manual_seed(31)
+    sets = [[(torch.randn(s, generator=gen) * 1e-3).to(DEV) for s in ((320, 700), (96, 200), (700, 320))]
+            for _ in range(6)]
+    want = [muon.orthogonalize(gs) for gs in sets]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [None] * len(sets)
+
+    def call(k, stream):
+        with torch.cuda.stream(stream):
+            got[k] = muon.orthogonalize(sets[k])
+
+    def check():
+        torch.cuda.synchronize()
+        for k, (xs, ys) in enumerate(zip(got, want)):
+            assert all(torch.equal(x, y) for x, y in zip(xs, ys)), k
+
+    for k in range(len(sets)):
+        call(k, streams[k % 2])
+    check()
+    for own in (True, False):
+        got[:] = [None] * len(sets)
+        threads = [threading.Thread(target=lambda t=t: [call(k, streams[t if own else 0])
+                                                        for k in range(t, len(sets), 2)])
+                   for t in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        check()
+
+
+def test_a_dropped_step_and_its_retry_on_another_stream():
+    """A hybrid step that raises leaves its first products queued on its stream: the next step, on
+    another one, waits for them before it writes the same workspace."""
+    class Model(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.a, self.b = nn.Linear(1024, 1536, bias=False), nn.Linear(1536, 1024, bias=False)
+
+    torch.manual_seed(2)
+    model = Model().to(DEV)
+    other = copy.deepcopy(model)
+    oa, ob = muon.HybridMuonAdamW(model), muon.HybridMuonAdamW(other)
+    gen = torch.Generator().manual_seed(3)
+    grads = [(torch.randn(p.shape, generator=gen) * 1e-3).to(DEV) for p in model.parameters()]
+    for m in (model, other):
+        for p, g in zip(m.parameters(), grads):
+            p.grad = g.clone()
+    model.b.weight.grad[3, 5] = float("nan")
+    with pytest.raises(FloatingPointError):
+        oa.step()
+    side = torch.cuda.Stream()
+    model.b.weight.grad = grads[1].clone()
+    side.wait_event(torch.cuda.current_stream().record_event())
+    with torch.cuda.stream(side):
+        oa.step()
+    ob.step()
+    torch.cuda.synchronize()
+    for p, q, g in zip(model.parameters(), other.parameters(), grads):
+        assert torch.equal(p, q)
+
+
 def test_transposed_flag_equals_passing_the_transposed_shape():
     """C ABI: a [c, r] matrix flagged transposed under (rows, cols) = (r, c) equals the
     same matrix passed unflagged as (c, r)."""
