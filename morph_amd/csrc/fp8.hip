@@ -26,11 +26,15 @@
 // each per half of the wave's span.  A workgroup holds 4 waves / 16 blocks.
 //
 // Bound: HBM, with launches so short (57 MB for a [6144, 3072] FP16 weight) that they are
-// a third fill and drain.  The pack reads the weights non-temporally and the unpack
-// writes them so, each touched once; the bytes in between keep ordinary accesses, for the
-// transfer or the unpack that follows.  Median of 8 rounds over nine such weights: pack
-// 12.7 -> 11.7 us, unpack 13.5 -> 10.2 us.  Against that, non-temporal bytes too: pack
-// 11.6, unpack 11.9; 1, 2 or 8 waves per workgroup: within 3%.
+// a third fill and drain.  The pack reads the weights non-temporally: once packed they have
+// been sent.  Three such weights that no cache holds, packed and unpacked: 73.2 -> 66.1 us;
+// a weight that is used again right behind its pack pays (a product with 256 rows of it
+// 40 -> 44 us).  The bytes keep ordinary accesses, for the transfer or the unpack that
+// follows, and so do the unpacked weights, which the next kernel reads: written
+// non-temporally they leave the Infinity Cache, and the unpack saves 0.5 us (10.2 -> 9.7)
+// where its reader loses more: with a product of 256 rows 41.6 -> 47.0 us, 1024 rows
+// 49.1 -> 53.7, 4096 rows 139.2 -> 140.5, an elementwise pass 22.3 -> 23.9; a [3072, 6144]
+// weight with 256 rows 36.6 -> 44.2.  1, 2 or 8 waves per workgroup: within 3%.
 #include <type_traits>
 
 #include "common.h"
@@ -293,13 +297,13 @@ __global__ __launch_bounds__(kThreads) void unpack_kernel(const uint8_t* __restr
     if (i + 8 <= n && (reinterpret_cast<uintptr_t>(dst) + i * kBytes) % 16 == 0) {
       if constexpr (std::is_same_v<OT, F32>) {
         float* d = static_cast<float*>(dst) + i;
-        store_stream<true>(reinterpret_cast<f32x4*>(d), f32x4{y[0], y[1], y[2], y[3]});
-        store_stream<true>(reinterpret_cast<f32x4*>(d + 4), f32x4{y[4], y[5], y[6], y[7]});
+        *reinterpret_cast<f32x4*>(d) = f32x4{y[0], y[1], y[2], y[3]};
+        *reinterpret_cast<f32x4*>(d + 4) = f32x4{y[4], y[5], y[6], y[7]};
       } else {
         u32x4 v;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = from_float<OT>(y[2 * k]) | (from_float<OT>(y[2 * k + 1]) << 16);
-        store_stream<true>(reinterpret_cast<u32x4*>(static_cast<uint16_t*>(dst) + i), v);
+        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(dst) + i) = v;
       }
       continue;
     }
