@@ -406,6 +406,21 @@ int morph_gemm_nt_bf16(const uint16_t* P, const uint16_t* Q, const uint16_t* D, 
                        int64_t stride_ct, float alpha, float beta, int flags, void* stream);
 
 /*
+ * The tile edge (256, 128 or 64) that a product of this size runs on, by the rule the
+ * launches follow; M, N and K multiples of 64, flags as morph_gemm_nt_bf16; epilogue: 0 plain,
+ * 1 with D, 2 the Muon update that morph_muon_newton_schulz_finish carries.  Nothing is
+ * launched.  A negative status for other arguments.
+ */
+int morph_gemm_tile_edge(int64_t M, int64_t N, int64_t K, int64_t batch, int flags, int epilogue);
+
+/*
+ * What the Newton-Schulz chain of `count` matrices of [rows, cols] runs on: the multiple (256,
+ * 128 or 64) that min(rows, cols) and max(rows, cols) are padded to, or 0 when each matrix
+ * runs its whole chain in one workgroup.  A negative status for bad arguments.
+ */
+int morph_muon_pad_multiple(int64_t rows, int64_t cols, int count, int ns_steps);
+
+/*
  * One Muon matrix: FP32 row-major device buffers of shape [rows, cols], or
  * [cols, rows] when `transposed` is 1.  Both orientations have the same
  * Newton-Schulz operand (optimizer.py:15-17 transposes the taller one), so one
@@ -528,9 +543,9 @@ int morph_muon_newton_schulz_finish(const morph_muon_matrix* mats, int count, in
 
 /*
  * The same in two calls, for a caller whose step may still be dropped after prepare
- * (a flag it reads back): _ahead enqueues the chain's first products, as many as cover
- * about 100 us, so that the device works while the flag travels; they write the
- * workspace only.  _finish_rest, with the same count, rows, cols, hp and workspace,
+ * (a flag it reads back): _ahead enqueues the chain's first products, at least one and
+ * until they make about 100 us, so that the device works while the flag travels; they write
+ * the workspace only.  _finish_rest, with the same count, rows, cols, hp and workspace,
  * enqueues what is left of the chain and the update.  Both together give the bits of
  * morph_muon_newton_schulz_finish; without _finish_rest no parameter has changed and
  * the workspace is free for another prepare behind the products, in stream order: on

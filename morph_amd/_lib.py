@@ -31,8 +31,8 @@ EXPORTS = (
     "morph_adamw_table_dev", "morph_nonfinite_table", "morph_step_end", "morph_nonfinite_or_close",
     "morph_grad_partials", "morph_grad_accumulate", "morph_grad_accumulate_final_noalloc",
     "morph_sumsq_total", "morph_convert_f32", "morph_fp8_pack", "morph_fp8_unpack",
-    "morph_gemm_nt_bf16",
-    "morph_muon_workspace_bytes", "morph_muon_step", "morph_muon_orthogonalize",
+    "morph_gemm_nt_bf16", "morph_gemm_tile_edge",
+    "morph_muon_workspace_bytes", "morph_muon_pad_multiple", "morph_muon_step", "morph_muon_orthogonalize",
     "morph_muon_prepare", "morph_muon_newton_schulz", "morph_muon_finish",
     "morph_muon_finish_range", "morph_muon_newton_schulz_finish",
     "morph_muon_newton_schulz_ahead", "morph_muon_newton_schulz_finish_rest", "morph_host_copy",
@@ -156,6 +156,8 @@ def _load():
         "morph_fp8_unpack": ([vp, vp, i64, vp, i32, vp], i32),
         "morph_gemm_nt_bf16": ([vp, vp, vp, vp, vp] + [i64] * 14 +
                                [ctypes.c_float, ctypes.c_float, i32, vp], i32),
+        "morph_gemm_tile_edge": ([i64, i64, i64, i64, i32, i32], i32),
+        "morph_muon_pad_multiple": ([i64, i64, i32, i32], i32),
         "morph_muon_workspace_bytes": ([i64, i64, i32], ctypes.c_size_t),
         "morph_muon_step": ([ctypes.POINTER(MuonMatrix), i32, i64, i64,
                              ctypes.POINTER(MuonHP), vp, ctypes.c_size_t, vp], i32),

@@ -1141,6 +1141,16 @@ int morph::gemm_kn_apply(const uint16_t* P, const uint16_t* Q, int64_t M, int64_
 
 using namespace morph;
 
+extern "C" int morph_gemm_tile_edge(int64_t M, int64_t N, int64_t K, int64_t batch, int flags,
+                                    int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || epilogue < 0 || epilogue > 2 ||
+      (flags & ~(MORPH_GEMM_SYMMETRIC | MORPH_GEMM_Q_KN)))
+    return MORPH_EINVAL;
+  if (M % kGemmEdge || N % kGemmEdge || K % MORPH_GEMM_TILE_K) return MORPH_ERANGE;
+  constexpr Epilogue kinds[3] = {Epilogue::kPlain, Epilogue::kWithD, Epilogue::kUpdate};
+  return choose_tile(M, N, K, batch, (flags & MORPH_GEMM_SYMMETRIC) != 0, kinds[epilogue]).ts;
+}
+
 extern "C" int morph_gemm_nt_bf16(const uint16_t* P, const uint16_t* Q, const uint16_t* D,
                                   uint16_t* C, uint16_t* Ct, int64_t M, int64_t N, int64_t K,
                                   int64_t batch, int64_t ldp, int64_t ldq, int64_t ldd,

@@ -162,6 +162,12 @@ size_t workspace_bytes_for(int64_t rows, int64_t cols, int64_t count) {
   return make_layout(rows, cols, count, MORPH_GEMM_TILE_M).total;
 }
 
+static_assert(kSmallMaxMats >= kMaxMats, "a whole batch in one small launch");
+
+// Small operands run the one-workgroup-per-matrix kernels (muon_small.hip).  With no
+// iterations there is no chain: those keep the general passes.
+bool takes_small(int64_t m, int64_t n, int64_t steps) { return steps >= 1 && small_fits(m, n); }
+
 template <int kLanes = kBlock>
 __device__ __forceinline__ double block_sum(double x, double* lds) {
 #pragma unroll
@@ -587,6 +593,13 @@ extern "C" size_t morph_muon_workspace_bytes(int64_t rows, int64_t cols, int cou
   return workspace_bytes_for(rows, cols, count);
 }
 
+extern "C" int morph_muon_pad_multiple(int64_t rows, int64_t cols, int count, int ns_steps) {
+  if (rows <= 0 || cols <= 0 || count <= 0 || ns_steps < 0) return MORPH_EINVAL;
+  if (count > kMaxMats) return MORPH_ERANGE;
+  const int64_t m = std::min(rows, cols), n = std::max(rows, cols);
+  return takes_small(m, n, ns_steps) ? 0 : (int)pad_multiple(m, n, count);
+}
+
 namespace {
 
 struct Bufs {
@@ -665,14 +678,6 @@ MatPtrs pointers(const morph_muon_matrix* mats, int count, int64_t rows, int64_t
   return m;
 }
 
-static_assert(kSmallMaxMats >= kMaxMats, "a whole batch in one small launch");
-
-// Small operands run the one-workgroup-per-matrix kernels (muon_small.hip).  With no
-// iterations there is no chain: those keep the general passes.
-bool takes_small(const Layout& L, const morph_muon_hp* hp) {
-  return hp->ns_steps >= 1 && small_fits(L.m, L.n);
-}
-
 // mats (nullable): the batch's descriptors, needed by prepare and by an updating chain.
 SmallBatch small_batch(const Bufs& W, const morph_muon_matrix* mats, int count) {
   const Layout& L = W.L;
@@ -719,7 +724,7 @@ int prepare(const morph_muon_matrix* mats, int count, int64_t rows, int64_t cols
   if (rc || count == 0) return rc;
   const Layout& L = W.L;
   hipStream_t s = as_stream(stream);
-  if (takes_small(L, hp))
+  if (takes_small(L.m, L.n, hp->ns_steps))
     return small_prepare(small_batch(W, mats, count), orth_only, hp->momentum_weight,
                          hp->nesterov_weight, found_inf, s);
   int n_all, n_flat, n_tiled;
@@ -777,12 +782,13 @@ bool can_fuse_update(const morph_muon_matrix* mats, int count, const Layout& L) 
 
 // How many of a chain's products (three per iteration) may run before the caller knows
 // that the step stands: enough to cover its round trip to the host, about 60 us, by the
-// GEMM's cost rule, which a step that is dropped then wastes; never the last product, which
-// may carry the parameter update.  The one-launch chain of small matrices has none.
+// GEMM's cost rule, and at least one; a step that is dropped then wastes them (1.9 ms for
+// the first product of 42 matrices of 3072 x 6144).  Never the last product, which may carry
+// the parameter update.  The one-launch chain of small matrices has none.
 // Both halves of a chain count them anew, so they depend on shape, count and steps only.
 int64_t products_ahead(const Layout& L, int count, const morph_muon_hp* hp) {
   constexpr double kCoverUs = 100.0;
-  if (hp->ns_steps < 1 || takes_small(L, hp)) return 0;
+  if (hp->ns_steps < 1 || takes_small(L.m, L.n, hp->ns_steps)) return 0;
   const double us[3] = {gemm_us(L.mp, L.mp, L.np, count, true, false),
                         gemm_us(L.mp, L.mp, L.mp, count, true, true),
                         gemm_us(L.mp, L.np, L.mp, count, false, false)};
@@ -810,7 +816,7 @@ int newton_schulz(int count, int64_t rows, int64_t cols, const morph_muon_hp* hp
   const int64_t last = part == Part::kAhead ? ahead : 3 * (int64_t)hp->ns_steps;
   auto runs = [&](int64_t it, int p) { return 3 * it + p >= first && 3 * it + p < last; };
   if (first >= last) return MORPH_OK;
-  if (takes_small(L, hp))
+  if (takes_small(L.m, L.n, hp->ns_steps))
     return run_small_chain(W, fuse, count, hp,
                            fuse != nullptr ? SmallOut::kApply : SmallOut::kStore,
                            as_stream(stream));
@@ -913,7 +919,7 @@ int newton_schulz_finish(const morph_muon_matrix* mats, int count, int64_t rows,
   Bufs W;
   int rc = setup(mats, count, rows, cols, hp, workspace, workspace_bytes, true, false, &W);
   if (rc || count == 0) return rc;
-  if (hp->ns_steps >= 1 && (takes_small(W.L, hp) || can_fuse_update(mats, count, W.L)))
+  if (hp->ns_steps >= 1 && (takes_small(W.L.m, W.L.n, hp->ns_steps) || can_fuse_update(mats, count, W.L)))
     return newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, mats, part);
   rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream, nullptr, part);
   if (!rc) rc = finish(mats, count, rows, cols, hp, workspace, workspace_bytes, false, stream);
@@ -990,7 +996,7 @@ extern "C" int morph_muon_orthogonalize(const morph_muon_matrix* mats, int count
   Bufs W;
   rc = setup(mats, count, rows, cols, hp, workspace, workspace_bytes, true, false, &W);
   if (rc) return rc;
-  if (takes_small(W.L, hp))
+  if (takes_small(W.L.m, W.L.n, hp->ns_steps))
     return run_small_chain(W, mats, count, hp, SmallOut::kExtract, as_stream(stream));
   rc = newton_schulz(count, rows, cols, hp, workspace, workspace_bytes, stream);
   if (!rc) rc = finish(mats, count, rows, cols, hp, workspace, workspace_bytes, true, stream);

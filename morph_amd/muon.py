@@ -157,14 +157,30 @@ def ns_flops(rows, cols, count, steps=NS_STEPS):
 
 def ns_executed_flops(rows, cols, count, steps=NS_STEPS):
     """FLOPs the MFMAs execute: the symmetric products (A = X X^T, B' = c A A + b A + a I)
-    compute only the upper triangle of their 256 x 256 tiles, X' = B' X all of them; the
-    operands are zero-padded to tile multiples (Mp, Np).  An upper bound for small batches,
-    which run smaller tiles with less padding."""
+    compute only the upper triangle of their tiles, X' = B' X all of them, over operands that
+    are zero-padded, both as the library pads and tiles this batch.  In the one-workgroup
+    chain each wave of a symmetric product computes two 32 x 32 tiles."""
     m, n = min(rows, cols), max(rows, cols)
-    mp, np_ = -(-m // 256) * 256, -(-n // 256) * 256
-    t, tn = mp // 256, np_ // 256
-    macs = t * (t + 1) // 2 * 256 * 256 * (np_ + mp) + t * tn * 256 * 256 * mp
-    return 2 * count * steps * macs
+    if steps < 1 or count < 1:
+        return 0
+    if count > 64:  # the library takes 64 at a time
+        return sum(ns_executed_flops(rows, cols, min(64, count - k), steps)
+                   for k in range(0, count, 64))
+    L = lib()
+    u = L.morph_muon_pad_multiple(rows, cols, count, steps)
+    check(min(u, 0))
+    mp, np_ = -(-m // (u or 32)) * (u or 32), -(-n // (u or 32)) * (u or 32)
+    if u == 0:
+        tiles = {32: 2, 64: 4, 96: 6, 128: 12}[mp] * 32 * 32
+        return 2 * count * steps * (tiles * (np_ + mp) + mp * mp * np_)
+
+    def upper(k, epilogue):  # elements of the tiles of a symmetric product over k
+        edge = L.morph_gemm_tile_edge(mp, mp, k, count, _lib.GEMM_SYMMETRIC, epilogue)
+        check(min(edge, 0))
+        t = mp // edge
+        return t * (t + 1) // 2 * edge * edge
+
+    return 2 * count * steps * (upper(np_, 0) * np_ + upper(mp, 1) * mp + mp * mp * np_)
 
 
 def _batch(mats, rows, cols, stream, workspaces, index):
@@ -208,8 +224,8 @@ def _finish_range(batch, first, n, stream):
 
 
 def _chains_ahead(batches, stream):
-    """The first products of every batch's chain, about 100 us of each; they write the
-    workspaces only."""
+    """The first products of every batch's chain, at least one and until they make about
+    100 us; they write the workspaces only."""
     L, sh = lib(), stream_handle(stream)
     for _, count, rows, cols, hp, ws in batches:
         check(L.morph_muon_newton_schulz_ahead(count, rows, cols, ctypes.byref(hp),
