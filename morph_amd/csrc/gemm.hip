@@ -845,7 +845,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const GemmApply* ap
     // 200 x 96 gradient 201 -> 190 us, 42 matrices of 3072 x 6144 39.1 -> 38.8 ms a step).
     //
     // Prologue: P0 Q0 P1 in full and the first half of Q1 (slots 0..3), then
-    // stage 0 is waited for and its first fragments read.
+    // stage 0 is waited for and its first fragments read.  (One stage or two come to the
+    // 128 edge only: choose_tile's costs give the 256 edge three at least.)
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) issue_load(false, 0, 0, j);
 #pragma unroll

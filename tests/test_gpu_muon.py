@@ -67,13 +67,36 @@ def test_gemm_q_kn_equals_the_nt_form_bit_for_bit(b, M, N, K):
     assert ((C - exact).abs() <= 2 ** -8 * exact.abs() + 1e-6 * K * mag + 1e-30).all()
 
 
-@pytest.mark.parametrize("M,N,K,batches", [(512, 512, 4096, (3, 12, 64)), (256, 512, 320, (2, 300)),
-                                           (256, 256, 192, (1, 512)), (256, 256, 128, (1, 512))])
-def test_gemm_tile_edges_give_the_same_bits(M, N, K, batches):
+ALL = {64, 128, 256}
+
+
+def tile_edge(M, N, K, batch, symmetric=False, epilogue=0):
+    from morph_amd import _lib
+    return _lib.lib().morph_gemm_tile_edge(M, N, K, batch, int(symmetric), epilogue)
+
+
+@pytest.mark.parametrize("M,N,K,reached", [
+    (512, 512, 4096, (ALL, ALL, ALL, ALL)), (256, 512, 320, (ALL, {64, 128}, {64, 128}, {64, 128})),
+    (256, 1024, 192, (ALL, {64}, {64, 128}, {64})), (256, 256, 192, (ALL, {64}, {64, 128}, {64})),
+    (512, 512, 256, (ALL, {64, 128}, {64, 128, 256}, {64, 128})),
+    (256, 256, 128, ({64, 128}, {64}, {64, 128}, {64})), (256, 256, 64, ({64, 128}, {64}, {64}, {64})),
+    (768, 768, 64, ({64, 128}, {64}, {64, 128}, {64}))])
+def test_gemm_tile_edges_give_the_same_bits(M, N, K, reached):
     """The batch decides the tile edge (64, 128 or 256: fewer tiles, smaller ones), never the
     bits: every output is one accumulator's sum over K in the same order, rounded once.  The
     smallest batch is checked against the float64 product, the larger ones against it; with
-    and without D, factors and Ct, [K, N] operands, and symmetric with mirror tiles."""
+    and without D, factors and Ct, [K, N] operands, and symmetric with mirror tiles.  The
+    batches are the smallest that the rule gives each edge; reached: the edges it gives plain
+    products, products with D, symmetric ones, and symmetric ones with D, up to 256 of them."""
+    kinds = [dict(), dict(epilogue=1), dict(symmetric=True), dict(symmetric=True, epilogue=1)]
+    batches = set()
+    for kw, edges in zip(kinds, reached):
+        first = {}
+        for b in range(1, 257):
+            first.setdefault(tile_edge(M, M if "symmetric" in kw else N, K, b, **kw), b)
+        assert set(first) == edges, kw
+        batches.update(first.values())
+    batches = sorted(batches)
     P, Q, D = rand_bf16((4, M, K), 1), rand_bf16((4, N, K), 2), rand_bf16((4, M, N), 3)
     S = rand_bf16((4, M, M), 4)
     forms = {}
@@ -100,11 +123,29 @@ def test_gemm_tile_edges_give_the_same_bits(M, N, K, batches):
     assert torch.equal(forms["sym"][0], forms["sym"][0].t())
 
 
-@pytest.mark.parametrize("shape,counts", [((330, 700), (1, 32, 64)), ((900, 450), (1, 8, 33)),
-                                          ((70, 45), (1, 40)), ((256, 320), (1, 64))])
+def muon_plan(shape, count, steps=5):
+    """What a batch runs on: its padding, the edges of A, B' and X', and of the product that
+    carries the update (None: padded operands, the finish pass); (0,): one workgroup each."""
+    from morph_amd import _lib
+    m, n = min(shape), max(shape)
+    u = _lib.lib().morph_muon_pad_multiple(m, n, count, steps)
+    if u == 0:
+        return (0,)
+    mp, np_ = -(-m // u) * u, -(-n // u) * u
+    update = tile_edge(mp, np_, mp, count, epilogue=2) if (mp, np_) == (m, n) else None
+    return (u, tile_edge(mp, mp, np_, count, True), tile_edge(mp, mp, mp, count, True, 1),
+            tile_edge(mp, np_, mp, count), update)
+
+
+@pytest.mark.parametrize("shape,counts", [((330, 700), (1, 30, 64)), ((900, 450), (1, 8, 33)),
+                                          ((70, 45), (1, 40)), ((256, 1024), (1, 14, 61)),
+                                          ((1000, 1200), (1, 5, 22))])
 def test_padding_and_tiles_do_not_change_the_bits(shape, counts):
     """A matrix's Newton-Schulz result, alone or among many: the batch's size decides how far
-    the operands are padded (64, 128 or 256) and the tile edges, and none of it the bits."""
+    the operands are padded (64, 128 or 256) and the tile edges, and none of it the bits; the
+    batches here all run on another plan, but for the one-workgroup chains of (70, 45)."""
+    plans = {muon_plan(shape, c) for c in counts}
+    assert len(plans) == (1 if shape == (70, 45) else len(counts)), plans
     gen = torch.Generator().manual_seed(9)
     gs = [(torch.randn(shape, generator=gen) * 1e-3).to(DEV) for _ in range(max(counts))]
     ref = [muon.orthogonalize(g) for g in gs[:3]]
@@ -359,15 +400,14 @@ def on_device(t, offset):
     ((300, 100), 0), ((70, 45), 0), ((300, 1), 0), ((4100, 1024), 0), ((4096, 640), 0),
     ((256, 640), 1), ((640, 256), 1), ((640, 256), 2), ((512, 768), 0), ((768, 512), 0)])
 def test_muon_step_elementwise_bitexact(shape, offset):
-    """momentum/Nesterov and the master update match the oracle bit for bit: the flat
-    passes (X in the stored layout: (128, 256) whole blocks, (100, 300) a partial last
-    block, (45, 70) rows not a multiple of 4, (96, 96) square, (1, 300) a single row) and
-    the transposing tile passes ((300, 100) and (70, 45) partial tiles only, (300, 1) a
-    single column, (4100, 1024) whole tiles and a partial last band, (4096, 640) whole
-    momentum tiles and a partial last column of apply tiles); with `offset`, parameter,
-    momentum and gradient start off a 16-byte boundary, so every pass takes its
-    element-wise path.  (512, 768) and (768, 512) have no operand padding: their update
-    rides on the last Newton-Schulz product's epilogue (morph_muon_newton_schulz_finish)."""
+    """momentum/Nesterov and the master update match the oracle bit for bit: the
+    one-workgroup kernels ((128, 256), (100, 300), (96, 96) and (1, 300) stored as X is,
+    (300, 100) transposed, (45, 70), (70, 45) and (300, 1) with rows that are no multiple of 4),
+    the transposing tile passes ((4100, 1024) whole tiles and a partial last band, with the
+    finish pass; (4096, 640) whole momentum tiles), and the flat passes and both with the
+    update on the last product's epilogue ((512, 768), (768, 512)).  With `offset`, parameter,
+    momentum and gradient start off a 16-byte boundary: (256, 640) and (640, 256) have no
+    padding, but the update takes the flat and the transposing finish pass."""
     from oracle import reference as R
     gen = torch.Generator().manual_seed(7)
     p0 = torch.randn(shape, generator=gen) * .02
@@ -588,19 +628,22 @@ def test_hybrid_state_dict_roundtrip():
         assert torch.equal(p, q), n
 
 
-@pytest.mark.parametrize("rows,cols,steps", [(256, 512, 5), (512, 256, 5), (512, 768, 2),
-                                             (768, 512, 1), (192, 320, 5), (320, 192, 1)])
-def test_update_in_the_last_product_equals_the_finish_pass(rows, cols, steps):
+@pytest.mark.parametrize("rows,cols,steps,edge", [
+    (256, 512, 5, 64), (512, 256, 5, 64), (512, 768, 2, 64), (768, 512, 1, 64), (192, 320, 5, 64),
+    (320, 192, 1, 64), (768, 2048, 5, 128), (2048, 768, 1, 128), (3072, 6144, 1, 256),
+    (6144, 3072, 2, 256), (330, 700, 5, None), (700, 330, 1, None)])
+def test_update_in_the_last_product_equals_the_finish_pass(rows, cols, steps, edge):
     """morph_muon_newton_schulz_finish carries the master update in the last X' = B' X
-    product's epilogue when the operand has no padding -- both orientations in one batch,
-    so the epilogue writes p rows from the tile's rows and from its columns, scale
-    sqrt(max(1, r/c)) per matrix; with steps == 1 the last product is also the first,
-    which carries 1/den -- and falls back to the finish pass otherwise ((192, 320),
-    (320, 192)).  Either way parameters and momenta are bit-identical to
+    product's epilogue when the operand has no padding, on each tile edge -- both
+    orientations in one batch, so the epilogue writes p rows from the tile's rows and from
+    its columns, scale sqrt(max(1, r/c)) per matrix; with steps == 1 the last product is also
+    the first, which carries 1/den -- and falls back to the finish pass otherwise ((330, 700),
+    (700, 330)).  Either way parameters and momenta are bit-identical to
     prepare + newton_schulz + finish."""
     import ctypes
     from morph_amd import _lib
     L = _lib.lib()
+    assert muon_plan((rows, cols), 4)[-1] == edge
     gen = torch.Generator().manual_seed(rows + cols + steps)
     shapes = [(rows, cols), (cols, rows), (rows, cols), (cols, rows)]
     p0 = [torch.randn(s, generator=gen) * .02 for s in shapes]
@@ -637,11 +680,12 @@ def test_update_in_the_last_product_equals_the_finish_pass(rows, cols, steps):
 
 
 @pytest.mark.parametrize("rows,cols,steps", [(256, 512, 5), (512, 256, 1), (192, 320, 5),
-                                             (1536, 3072, 5), (96, 200, 5), (256, 256, 0)])
+                                             (1536, 3072, 5), (96, 200, 5), (256, 256, 0),
+                                             (330, 700, 5), (700, 330, 1), (900, 2050, 5)])
 def test_chain_in_two_calls_equals_one(rows, cols, steps):
     """morph_muon_newton_schulz_ahead writes no parameter; with _finish_rest behind it the bits
-    are those of newton_schulz_finish (with padding and without, a chain that the first
-    call runs to its last product, one whose first product is cover enough, the
+    are those of newton_schulz_finish (without padding and with it, where the finish pass
+    follows the rest of the chain; a chain that the first call runs to its last product, one whose first product is cover enough, the
     one-launch chain, no iterations), and a step dropped in between leaves nothing behind."""
     import ctypes
     from morph_amd import _lib
