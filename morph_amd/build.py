@@ -28,6 +28,7 @@ FLAGS = [
     "-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{ROOT / 'include'}",
+    "-Werror=align-mismatch",  # a pointer passed on with a larger alignment than its type has
 ]
 
 

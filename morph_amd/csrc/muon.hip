@@ -215,15 +215,16 @@ __device__ __forceinline__ void flag_nonfinite(uint32_t* found_inf, bool bad) {
 
 // Four consecutive elements of a stored row, `left` of them inside the row: one 16-byte
 // access when all are (4-byte aligned: rows of any length and views at any offset; the
-// hardware takes 16-byte accesses at any multiple of 4), else one element at a time.
+// hardware takes 16-byte accesses at any multiple of 4), else one element at a time.  The
+// accesses keep the row type: a template argument would drop its alignment.
 typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ f32x4 load_row4(const float* p) {
-  return load_stream<true>(reinterpret_cast<const f32x4_row*>(p));
+  return __builtin_nontemporal_load(reinterpret_cast<const f32x4_row*>(p));
 }
 
 __device__ __forceinline__ void store_row4(float* p, const f32x4& v) {
-  store_stream<true>(reinterpret_cast<f32x4_row*>(p), (f32x4_row)v);
+  __builtin_nontemporal_store((f32x4_row)v, reinterpret_cast<f32x4_row*>(p));
 }
 
 __device__ __forceinline__ f32x4 load_row4(const float* p, int64_t left) {
