@@ -35,11 +35,15 @@ const at::Tensor* plain_tensor(PyObject* o) {
   return t.defined() && plain(t) ? &t : nullptr;
 }
 
+// Whether t is n contiguous elements of `type`.
+bool holds(const at::Tensor& t, at::ScalarType type, int64_t n) {
+  return t.numel() == n && t.scalar_type() == type && t.is_contiguous();
+}
+
 // Whether o is still the n floats at `address` that a descriptor points at.
 bool still_at(PyObject* o, const void* address, int64_t n) {
   const at::Tensor* t = plain_tensor(o);
-  return t != nullptr && t->numel() == n && t->scalar_type() == at::kFloat && t->is_contiguous() &&
-         t->const_data_ptr() == address;
+  return t != nullptr && holds(*t, at::kFloat, n) && t->const_data_ptr() == address;
 }
 
 // A list's or tuple's items, borrowed; false for anything else.
@@ -93,6 +97,7 @@ class StepPlan {
     const size_t n = present_.size();
     numels_.resize(n);
     ptrs_.resize(n);
+    grads_.resize(n);
     for (size_t k = 0; k < n; ++k) {
       const int64_t i = present_[k];
       if (i < 0 || i >= (int64_t)params_.size() || (k > 0 && i <= present_[k - 1]))
@@ -124,8 +129,6 @@ class StepPlan {
     const Py_ssize_t total = PyList_GET_SIZE(params_.ptr());
     if (!given.ok || (!own && given.n != total)) return false;
     if (outs.n != 0 && outs.n != total) return false;
-    std::vector<at::Tensor> held;
-    held.reserve(present_.size());
     Py_ssize_t i = 0, in_state = 0;
     size_t k = 0;
     for (Py_ssize_t g = 0; g < gs.n; ++g) {
@@ -140,21 +143,18 @@ class StepPlan {
         PyObject *owner = nullptr, *moments = nullptr;  // borrowed
         if (!PyDict_Next(state.ptr(), &in_state, &owner, &moments) || owner != po) return false;
         const bool want = k < present_.size() && present_[k] == i;
-        at::Tensor grad;
+        const at::Tensor* grad = nullptr;
         if (own) {
           const at::Tensor* p = plain_tensor(po);
           if (p == nullptr) return false;
-          grad = p->unsafeGetTensorImpl()->grad();
-          if (grad.defined() != want) return false;
-          if (want && !plain(grad)) return false;
+          grad = &p->unsafeGetTensorImpl()->grad();
+          if (grad->defined() != want) return false;
+          if (want && !plain(*grad)) return false;
         } else {
           PyObject* go = given.at(i);
           if ((go == Py_None) == want) return false;
-          if (want) {
-            const at::Tensor* t = plain_tensor(go);
-            if (t == nullptr) return false;
-            grad = *t;
-          }
+          if (want) grad = plain_tensor(go);
+          if (want && grad == nullptr) return false;
         }
         if (!want) continue;
         static PyObject* const first = PyUnicode_InternFromString("exp_avg");
@@ -164,8 +164,8 @@ class StepPlan {
             !still_at(PyDict_GetItemWithError(moments, first), d.exp_avg, d.numel) ||
             !still_at(PyDict_GetItemWithError(moments, second), d.exp_avg_sq, d.numel))
           return false;
-        if (grad.layout() != at::kStrided || grad.device() != device_ ||
-            grad.scalar_type() != type_ || grad.numel() != numels_[k] || !grad.is_contiguous())
+        if (grad->layout() != at::kStrided || grad->device() != device_ ||
+            !holds(*grad, type_, d.numel))
           return false;
         void* out = nullptr;
         if (outs.n != 0) {
@@ -173,20 +173,29 @@ class StepPlan {
           if (o == nullptr) return false;
           out = o->data_ptr();
         }
-        if (out != desc_[k].out) return false;
-        ptrs_[k] = grad.data_ptr();
-        held.push_back(std::move(grad));
+        if (out != d.out) return false;
+        ptrs_[k] = grad->const_data_ptr();
+        grads_[k] = grad;
         ++k;
       }
     }
     if (i != total || k != present_.size()) return false;
-    for (k = 0; k < present_.size(); ++k) desc_[k].grad = ptrs_[k];
-    held_.swap(held);
+    std::vector<at::Tensor> dropped;  // freed when all is done: that can run any code
+    held_.resize(present_.size());
+    for (k = 0; k < present_.size(); ++k) {
+      desc_[k].grad = ptrs_[k];
+      if (held_[k].is_same(*grads_[k])) continue;
+      dropped.push_back(std::move(held_[k]));
+      held_[k] = *grads_[k];
+    }
     return true;
   }
 
   // Lets go of the last match's gradients.
-  void release() { held_.clear(); }
+  void release() {
+    std::vector<at::Tensor> dropped;
+    dropped.swap(held_);
+  }
 
   // The step's launches on `stream` after match(): the detector (unless `checked`; with the
   // previous step's close when prev_list is not 0), then AdamW.  The status of the first
@@ -236,6 +245,7 @@ class StepPlan {
   Entries fn_;
   std::vector<int64_t> numels_;
   std::vector<const void*> ptrs_;
+  std::vector<const at::Tensor*> grads_;  // during a match
   std::vector<at::Tensor> held_;
   bool closed_ = false;
   at::Device device_{at::kCPU};
