@@ -610,6 +610,9 @@ extern "C" int morph_adamw_table_dev(const void* d_table, const morph_adamw_tens
   a.state = d_state;
   hipStream_t s = as_stream(stream);
   int64_t block = 0;
+  bool first_launch = true;
+  int last = count - 1;  // the last tensor with elements: its launch stamps the stop event
+  while (last >= 0 && tensors[last].numel == 0) --last;
   for (int r0 = 0; r0 < count; r0 += kTableRefs) {
     const int r1 = count - r0 < kTableRefs ? count : r0 + kTableRefs;
     a.first_row = r0;
@@ -624,10 +627,11 @@ extern "C" int morph_adamw_table_dev(const void* d_table, const morph_adamw_tens
       grad_bytes += x.numel * gb;
     }
     a.reverse = grad_bytes > kReverseAboveBytes ? 1 : 0;
-    const Stamps ev{r0 == 0 ? static_cast<hipEvent_t>(start_event) : nullptr,
-                    r1 == count ? static_cast<hipEvent_t>(stop_event) : nullptr};
     block += blocks;
     if (blocks == 0) continue;
+    const Stamps ev{first_launch ? static_cast<hipEvent_t>(start_event) : nullptr,
+                    last < r1 ? static_cast<hipEvent_t>(stop_event) : nullptr};
+    first_launch = false;
     const uint32_t* skip = &d_state->found_inf[slot];
     switch (grad_dtype) {
       case MORPH_DTYPE_F32: rc = launch_table_out<F32>(out_dtype, a, d_table, count, (int)blocks, skip, s, ev); break;

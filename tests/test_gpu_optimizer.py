@@ -633,6 +633,27 @@ def test_many_tensors_can_be_captured_after_one_step():
     assert all(torch.equal(x, y) for x, y in zip(*runs))
 
 
+@pytest.mark.parametrize("empty", [range(400, 450), range(0, 400), range(0, 450)],
+                         ids=["last launch", "first launch", "all"])
+def test_a_table_step_is_stamped_around_its_launches(empty):
+    """The start event is stamped by the first launch of a step that has elements, the stop event
+    by the last: 450 tensors over the descriptor table, 400 to a launch, those of one empty."""
+    from morph_amd import kernels
+    n = 1 << 14
+    ps = [torch.zeros(0 if i in empty else n, device=DEV) for i in range(450)]
+    opt = FusedAdamW(ps, lr=1e-3)
+    gs = [torch.ones_like(p) for p in ps]
+    opt.step(gs)
+    assert opt._cache[0]._table is not None
+    opt.dispatch_timer = kernels.DispatchTimer(2)
+    opt.step(gs)
+    opt.step(gs)
+    torch.cuda.synchronize()
+    if len(empty) < 450:
+        assert all(1e-3 < ms < 50 for ms in opt.dispatch_timer.elapsed_ms())
+    assert all(torch.isfinite(p).all() for p in ps)
+
+
 @pytest.mark.parametrize("count", [5, 60])
 def test_native_steps_equal_python_steps(count):
     """From a batch's second step on the launches go out natively (hostpath.cpp).  A sequence that
