@@ -41,8 +41,7 @@ class BiasTables:
 
     def used_on(self, stream):
         """Note that work reading the current tables is enqueued on `stream`."""
-        if stream != torch.cuda.current_stream(self.device):
-            self._streams.add(stream)
+        self._streams.add(stream)
 
     def ensure(self, t_max):
         if t_max <= self.length:

@@ -152,6 +152,7 @@ class FusedAdamW:
         self._cache = None
         self._plan = None       # hostpath.StepPlan over the cached batch, from its second step on
         self._plan_key = None   # the cache key it was built for
+        self._read_on = self._read_list = None  # the stream that is noted for them, and the list
         self._consts = None     # (hyperparameters, constants, schedules, table limit) of the groups
         if self._staging is None:
             _lib.hostpath()     # a missing build fails here (CPU masters have no plan)
@@ -243,6 +244,7 @@ class FusedAdamW:
         key = (float(betas[0]), float(betas[1]))
         if key not in self._tables:
             self._tables[key] = BiasTables(key[0], key[1], self.device)
+            self._read_on = None
         return self._tables[key]
 
     def _places(self, present):
@@ -317,7 +319,9 @@ class FusedAdamW:
             hps.append(adamw_constants(lr=group["lr"], beta1=beta1, beta2=beta2, eps=group["eps"],
                                        weight_decay=group["weight_decay"], step=1))
             table = self._table(group["betas"])
-            table.ensure(need)
+            if need > table.length:
+                table.ensure(need)
+                self._read_on = None
             scheds.append(table.sched(group["lr"]))
             limit = table.length if limit is None else min(limit, table.length)
         hps = (_lib.AdamwHP * len(hps))(*hps)
@@ -481,12 +485,13 @@ class FusedAdamW:
         events = self.dispatch_timer.next() if self.dispatch_timer is not None else None
         ctl = self._ctl
         slot = self._slot
-        current = torch.cuda.current_stream(self.device)
-        s = stream or current
-        if s != current:
+        s = stream or torch.cuda.current_stream(self.device)
+        if self._read_on != s or self._read_list is not clock_list:
+            # the tables and the clock list may have been allocated on another stream
             for table in self._tables.values():
                 table.used_on(s)
-            clock_list.record_stream(s)  # allocated on the current stream, read on `s`
+            clock_list.record_stream(s)
+            self._read_on, self._read_list = s, clock_list
         if self._pending is not None and self._pending[2] != s:
             # the previous step ran on another stream: close it there, and order
             # this step after that close

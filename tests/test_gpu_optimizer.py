@@ -1091,6 +1091,33 @@ def test_after_the_minimum_scale_raise_the_optimizer_goes_on():
     assert opt.state[w]["step"] == 2
 
 
+def test_memory_read_under_another_current_stream_is_noted(monkeypatch):
+    """An optimizer's clock list and bias tables are allocated on the stream that is current at
+    its first step; steps under another current stream read them there, so the allocator is
+    told: a list replaced by another set of gradients is not handed out under that work."""
+    noted = []
+    real = torch.Tensor.record_stream
+    monkeypatch.setattr(torch.Tensor, "record_stream",
+                        lambda t, s: (noted.append((t.data_ptr(), s)), real(t, s))[1])
+    ps = [torch.zeros(100, device=DEV) for _ in range(2)]
+    gs = [torch.ones(100, device=DEV) for _ in range(2)]
+    opt = FusedAdamW(ps, lr=1e-3)
+    opt.step(gs)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            opt.step(gs)
+    clock_list, table = opt._cache[1], opt._tables[(.9, .999)]
+    assert (clock_list.data_ptr(), side) in noted and side in table._streams
+    old = (table.bc1.data_ptr(), side)
+    opt._bound = 4096
+    with torch.cuda.stream(side):
+        opt.step(gs)
+    assert old in noted and side in table._streams
+    opt.resolve()
+
+
 def test_bias_tables_grow_past_4096_steps_on_a_side_stream():
     """The bias-correction tables double at step 4097; the old ones stay valid for the
     side stream's queued launches.  Result bit-exact against the oracle."""
