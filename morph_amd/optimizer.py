@@ -486,7 +486,7 @@ class FusedAdamW:
         ctl = self._ctl
         slot = self._slot
         s = stream or torch.cuda.current_stream(self.device)
-        if self._read_on != s or self._read_list is not clock_list:
+        if self._read_on is None or self._read_on != s or self._read_list is not clock_list:
             # the tables and the clock list may have been allocated on another stream
             for table in self._tables.values():
                 table.used_on(s)
