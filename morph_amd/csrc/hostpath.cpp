@@ -252,9 +252,24 @@ class StepPlan {
   at::ScalarType type_;
 };
 
+// Where each tensor of the list lies, its size and whether it is contiguous, for a key.
+py::bytes places(const py::list& tensors) {
+  std::vector<int64_t> out;
+  out.reserve(2 * tensors.size());
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(tensors.ptr()); ++i) {
+    PyObject* o = PyList_GET_ITEM(tensors.ptr(), i);
+    if (!THPVariable_Check(o)) throw py::type_error("places() takes tensors");
+    const at::Tensor t = THPVariable_Unpack(o);
+    out.push_back(reinterpret_cast<int64_t>(t.const_data_ptr()));
+    out.push_back(t.is_contiguous() ? t.numel() : ~t.numel());
+  }
+  return py::bytes(reinterpret_cast<const char*>(out.data()), out.size() * sizeof(int64_t));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_hostpath, m) {
+  m.def("places", &places);
   py::class_<StepPlan>(m, "StepPlan")
       .def(py::init<py::list, std::vector<int64_t>, uint64_t, int, int, uint64_t, uint64_t, uint64_t,
                     std::vector<uint64_t>>())

@@ -250,14 +250,17 @@ class FusedAdamW:
     def _places(self, present):
         """Where the listed masters and moments lie: a caller may move a parameter (p.data) or
         replace a moment in self.state between steps."""
-        masters = [self._dev[i] for i in present]
-        states = [self.state[p] for p in self._listed(present)]
-        return (tuple((p.data_ptr(), p.numel(), p.is_contiguous()) for p in masters),
-                tuple((s["exp_avg"].data_ptr(), s["exp_avg_sq"].data_ptr()) for s in states))
-
-    def _listed(self, present):
-        flat = self._flat()
-        return [flat[i][1] for i in present]
+        flat, items = self._flat(), list(self.state.items())
+        states = []
+        for i in present:  # the state is in the parameters' order: a lookup by them takes longer
+            own = i < len(items) and items[i][0] is flat[i][1]
+            states.append(items[i][1] if own else self.state[flat[i][1]])
+        tensors = [self._dev[i] for i in present]
+        for name in ("exp_avg", "exp_avg_sq"):
+            tensors += [s[name] for s in states]
+        if self._staging is None:
+            return _lib.hostpath().places(tensors)
+        return tuple(t.data_ptr() for t in tensors)  # the mirrors keep size and layout
 
     def _prepare(self, grads, present):
         """Descriptor batch, clock list and parameter groups for this set of tensors."""
@@ -271,7 +274,7 @@ class FusedAdamW:
                self._places(present))
         ptrs = tuple(grads[i].data_ptr() for i in present)
         if key != self._cache_key:
-            ps = self._listed(present)
+            ps = [flat[i][1] for i in present]
             if self._cache is not None and self._pending is not None:
                 # tensors that only the old batch still holds may be in use there
                 self._cache[0].used_on(self._pending[2])

@@ -213,6 +213,18 @@ def test_launch_says_whether_the_detector_went_out(detector, adamw, closed):
     assert c.plan.closed() == closed
 
 
+def test_places_tell_tensors_apart():
+    places = _lib.hostpath().places
+    t = torch.zeros(4, 6)
+    of = lambda *ts: places(list(ts))  # noqa: E731
+    assert of(t, t) == of(t, t.view(24)) and of(t) == of(torch.nn.Parameter(t))
+    others = [t[:2], t[1:], t.t(), torch.zeros(4, 6), t.view(-1)[::2], t[:0]]
+    assert len({of(t)} | {of(x) for x in others}) == 1 + len(others)
+    assert of(t, others[0]) != of(others[0], t) and of() == b""
+    with pytest.raises(TypeError):
+        of(t, None)
+
+
 def test_bad_plans_raise():
     p = [torch.zeros(3)]
     make = lambda present, entries=5: _lib.hostpath().StepPlan(  # noqa: E731
