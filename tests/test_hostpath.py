@@ -117,6 +117,14 @@ def test_anything_else_is_refused(change):
     assert not c.match(gs)
 
 
+def test_empty_views_of_a_larger_buffer_match():
+    c = Case()
+    empty = c.params[2]
+    empty.data = torch.zeros(9)[4:4]
+    c.state[empty] = dict(step=0, exp_avg=torch.zeros(8)[3:3], exp_avg_sq=torch.zeros(8)[8:])
+    assert c.match(c.grads())
+
+
 def test_other_containers_are_refused():
     c = Case()
     gs = c.grads()
