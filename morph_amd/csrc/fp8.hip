@@ -28,8 +28,8 @@
 // Bound: HBM, with launches so short (57 MB for a [6144, 3072] FP16 weight) that they are
 // a third fill and drain.  The pack reads the weights non-temporally: once packed they have
 // been sent.  Three such weights that no cache holds, packed and unpacked: 73.2 -> 66.1 us;
-// a weight that is used again right behind its pack pays (a product with 256 rows of it
-// 40 -> 44 us).  The bytes keep ordinary accesses, for the transfer or the unpack that
+// weights that the Infinity Cache holds pay (packed again and again 11.2 -> 12.7 us each), and
+// one that is used right behind its pack (a product with 256 rows of it 40 -> 44 us).  The bytes keep ordinary accesses, for the transfer or the unpack that
 // follows, and so do the unpacked weights, which the next kernel reads: written
 // non-temporally they leave the Infinity Cache, and the unpack saves 0.5 us (10.2 -> 9.7)
 // where its reader loses more: with a product of 256 rows 41.6 -> 47.0 us, 1024 rows

@@ -7,11 +7,14 @@
 // workgroup of 8 waves keeps both there: per iteration A = X X^T, B' = b A + c A A +
 // a I over A, X' = B' X over X, with a barrier between them.  Bound: LDS reads (a
 // 32 x 32 x 16 MFMA takes two fragments of 1 KiB; X' shares its fragments over the
-// wave's tiles).  One CU per matrix is enough up to m = 128: there an iteration costs
-// about what three launches do.
+// wave's tiles).  One CU per matrix is enough up to m = 128, whatever the batch (one of 64
+// matrices leaves the other CUs idle, and so do products of a tile or two).
 //
-// Measured, orthogonalize of one 200 x 96 gradient: 85 us a call (20 launches, 82 us of
-// kernels) -> 30.6 us (2 launches).
+// Measured, orthogonalize, us a call, the general products (on their 64 edge) -> this:
+// one gradient of 200 x 96 80 -> 30, of 128 x 128 78 -> 31, and at the limits of the LDS of
+// 128 x 480 80 -> 58, 96 x 736 82 -> 59, 64 x 1184 84 -> 63, 32 x 2496 107 -> 62; eight of
+// 128 x 480 96 -> 60; sixty-four of them 220 -> 173, sixty-four of 32 x 32 217 -> 167, both
+// then bound by the host.
 //
 // The bits are the general path's: 32x32x16 MFMAs over K in the same order (zero
 // padding adds nothing), the same scaling, fused multiply-adds and roundings.  Only
